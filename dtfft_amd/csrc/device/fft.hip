@@ -194,7 +194,13 @@ struct sched {
     static constexpr __device__ __host__ int span(int p) {  // L_p = product of radices before p
         return p == 0 ? 1 : span(p - 1) * radix(p - 1);
     }
-    // offset of pass p's twiddles in the table: sum over q < p of L_q * (R_q - 1)
+    // offset of pass p's twiddles in the table: sum over q < p of L_q * (R_q - 1).  Callers
+    // take it as a constexpr: evaluated at run time, its recursion is no longer inlined from the
+    // fourth pass on, and the kernel holds calls, a stack in scratch memory and the register
+    // budget of a call.  MI355X, run time -> constexpr: 384 x 210 x 320 FP64 X->Y pass
+    // (210 = 2 3 5 7) 239 -> 128 VGPRs, 422 -> 206 us; 512^3 FP32 R2R rows (4 4 4 4) 203 -> 94
+    // VGPRs (one -> two blocks per CU), 542 -> 301 us; 333-point FP32 lines by Bluestein
+    // (672 = 8 4 3 7) 707 -> 256 us.
     static constexpr __device__ __host__ int tw_off(int p) {
         return p == 0 ? 0 : tw_off(p - 1) + span(p - 1) * (radix(p - 1) - 1);
     }
@@ -263,6 +269,7 @@ struct fft_tile {
                                                 bool inv) {
         constexpr int R = S::radix(p);
         constexpr int L = S::span(p);
+        constexpr int TWO = S::tw_off(p);
         constexpr int NB = N / R;
         constexpr int IT = (NB + TPL - 1) / TPL;
         constexpr bool EXACT = (IT * TPL == NB);
@@ -302,7 +309,7 @@ struct fft_tile {
                 if (L > 1) {
 #pragma unroll
                     for (int r = 1; r < R; r++)
-                        v[it][r] = twmul(v[it][r], tw[S::tw_off(p) + k * (R - 1) + (r - 1)]);
+                        v[it][r] = twmul(v[it][r], tw[TWO + k * (R - 1) + (r - 1)]);
                 }
                 bfly<T, R>::run(v[it]);
                 const int base = (b - k) * R + k;
@@ -783,6 +790,7 @@ struct cols_dma {
     static __device__ __forceinline__ void pass(cx<T>* buf, const tw_t* twl, bool inv) {
         constexpr int R = S::radix(p);
         constexpr int L = S::span(p);
+        constexpr int TWO = S::tw_off(p);
         constexpr int NB = N / R;
         constexpr int IT = (NB + TPL - 1) / TPL;
         constexpr bool EXACT = (IT * TPL == NB);
@@ -810,7 +818,7 @@ struct cols_dma {
                 if (L > 1) {
 #pragma unroll
                     for (int r = 1; r < R; r++)
-                        v[it][r] = twmul(v[it][r], twl[S::tw_off(p) + k * (R - 1) + (r - 1)]);
+                        v[it][r] = twmul(v[it][r], twl[TWO + k * (R - 1) + (r - 1)]);
                 }
                 bfly<T, R>::run(v[it]);
                 const int base = (b - k) * R + k;
