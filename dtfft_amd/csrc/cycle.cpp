@@ -163,9 +163,10 @@ static int32_t make_group(const cycle_t* cy, const std::vector<stage_spec>& spec
 // Candidate tile shapes of a group for the autotuner, the default first: radix schedules of
 // the length (radix_schedules), threads per line of one or two butterflies of the largest
 // radix per pass, and the default's lines per block, halved and doubled.
-static std::vector<fft_config> group_candidates(int n, bool dbl, bool in_cols, bool out_cols, int effort) {
+static std::vector<fft_config> group_candidates(int n, bool dbl, bool in_cols, bool out_cols, int64_t lines,
+                                                int effort) {
     std::vector<fft_config> out;
-    const fft_config base = default_fft_config(n, dbl, in_cols, out_cols, in_cols && out_cols);
+    const fft_config base = default_fft_config(n, dbl, in_cols, out_cols, lines, INT64_MAX);
     out.push_back(base);
     const auto scheds = radix_schedules(n, effort >= DTFFT_HIP_EXHAUSTIVE ? 6 : 3);
     for (const auto& r : scheds) {
@@ -201,15 +202,17 @@ static int32_t tune_group(cycle_t* cy, const std::vector<stage_spec>& specs, con
                           bool in_cols, bool out_cols, void* scratch_in, void* scratch_out, fft_config& best) {
     const int n = (int)specs[members[0]].n;
     std::vector<int64_t> sig;
+    int64_t lines = 0;
     for (int g : members) {
         const stage_spec& q = specs[g];
+        lines += q.nl * q.nb;
         sig.insert(sig.end(), {q.nl, q.nb, q.in_ls, q.in_bs, q.in_ns, q.out_ls, q.out_bs, q.out_ns});
     }
     char kb[160];
     std::snprintf(kb, sizeof kb, "cyc|%d|%c|%d%d|%zu|%016llx", n, cy->dbl ? 'd' : 'f', (int)in_cols, (int)out_cols,
                   members.size(), (unsigned long long)fnv1a_ints(sig));
     const std::string key(kb);
-    best = default_fft_config(n, cy->dbl, in_cols, out_cols, in_cols && out_cols);
+    best = default_fft_config(n, cy->dbl, in_cols, out_cols, lines, INT64_MAX);
     std::string rec;
     if (tune_lookup(key, rec)) {
         int t, l, p;
@@ -223,7 +226,7 @@ static int32_t tune_group(cycle_t* cy, const std::vector<stage_spec>& specs, con
         return DTFFT_HIP_SUCCESS;
     }
     if (cy->effort < DTFFT_HIP_MEASURE || compile_only() || !scratch_in) return DTFFT_HIP_SUCCESS;
-    auto cands = group_candidates(n, cy->dbl, in_cols, out_cols, cy->effort);
+    auto cands = group_candidates(n, cy->dbl, in_cols, out_cols, lines, cy->effort);
     // compile the candidates side by side (hipRTC programs are independent)
     {
         std::vector<std::thread> pool;

@@ -13,8 +13,6 @@
 //     a linear convolution that a cyclic one of length M >= 2n - 1 holds exactly:
 //       X_k = c_k IDFT_M(DFT_M(a) DFT_M(b))_k,  a_j = x_j c_j (j < n, else 0),
 //       b_j = conj(c_j) for j < n, b_{M-j} = conj(c_j) for 0 < j < n, else 0.
-//     bh = DFT_M(b) / M is a table made once per (n, M); the inverse transform is
-//     conj(DFT_M(conj(.))), so both transforms run the forward passes.
 // KIND 0: C2C, complex in and out; the backward sign conjugates on load and store.
 // KIND 1: R2C, n reals in, n/2 + 1 complex out (forward).
 // KIND 2: C2R, n/2 + 1 complex in, n reals out (backward, FFTW c2r semantics: the input is
@@ -22,32 +20,140 @@
 //         Im X_{n/2} do not contribute).
 // Lines are addressed as in fft_tile, (l, b) with line start l * ls + b * bs, element
 // stride ns, in units of the element type of each side (reals for the real side).
-// Each block reads its lines whole before it writes, so in place is safe.
+// A block's last read of global memory precedes its first write (a barrier between), so in
+// place is safe.
+// bh = DFT_M(b) / M is a table made once per (n, M); the inverse transform is
+// conj(DFT_M(conj(.))), so both transforms run forward passes.  The second one runs the radices
+// in reverse: the last pass of the first transform (radix R, span M / R) leaves elements
+// b + s M / R in the registers of butterfly b, and the first pass of the second reads the same
+// ones, so product and both butterflies take one trip through LDS.  The first pass reads global
+// memory (its elements past n are zeros), the last one writes it: M = R0 R1 costs two LDS
+// exchanges, M = R0 R1 R2 four.
 #include "fft.hip"
 
-template <typename T, class S, int TPL, int LPB, int PAD, int KIND, bool CHIRP>
+namespace dtfft {
+// Passes of S with N / R butterflies spread over TPL threads of a line, elements taken from and
+// given to functors: load(line, n) and store(line, n, value).
+template <typename T, class S, int TPL, int LPB>
+struct any_passes {
+    typedef typename tw_of<T>::type tw_t;
+    static constexpr int NT = TPL * LPB;
+
+    template <bool COLS>
+    static __device__ __forceinline__ void map(int& line, int& j) {
+        if (COLS) { line = threadIdx.x % LPB; j = threadIdx.x / LPB; }
+        else { line = threadIdx.x / TPL; j = threadIdx.x % TPL; }
+    }
+
+    // pass p; BAR: a barrier between the last load and the first store (in place in LDS)
+    template <int p, bool COLS, bool BAR, class Load, class Store>
+    static __device__ __forceinline__ void run(const tw_t* __restrict__ tw, const Load& load, const Store& store) {
+        constexpr int R = S::radix(p), L = S::span(p), TWO = S::tw_off(p);
+        constexpr int NB = S::N / R, IT = (NB + TPL - 1) / TPL;
+        int line, j;
+        map<COLS>(line, j);
+        cx<T> v[IT][R];
+#pragma unroll
+        for (int it = 0; it < IT; it++) {
+            const int b = j + it * TPL;
+            if (IT * TPL == NB || b < NB) {
+#pragma unroll
+                for (int r = 0; r < R; r++) v[it][r] = load(line, b + r * NB);
+            }
+        }
+        if (BAR) __syncthreads();
+#pragma unroll
+        for (int it = 0; it < IT; it++) {
+            const int b = j + it * TPL;
+            if (IT * TPL == NB || b < NB) {
+                const int k = b % L;
+                if (L > 1) {
+#pragma unroll
+                    for (int r = 1; r < R; r++) v[it][r] = twmul(v[it][r], tw[TWO + k * (R - 1) + (r - 1)]);
+                }
+                bfly<T, R>::run(v[it]);
+#pragma unroll
+                for (int s = 0; s < R; s++) store(line, (b - k) * R + k + s * L, v[it][s]);
+            }
+        }
+    }
+
+    // The last pass of S, the product with bh and the conjugation, and the first pass of the
+    // reversed schedule, in place in LDS (line stride LD).
+    template <int LD>
+    static __device__ __forceinline__ void turn(const tw_t* __restrict__ tw, const tw_t* __restrict__ bh, cx<T>* lds) {
+        constexpr int p = S::NP - 1;
+        constexpr int R = S::radix(p), TWO = S::tw_off(p);
+        constexpr int NB = S::N / R, IT = (NB + TPL - 1) / TPL;
+        static_assert(S::span(p) == NB, "the last pass");
+        int line, j;
+        map<false>(line, j);
+        cx<T> v[IT][R];
+#pragma unroll
+        for (int it = 0; it < IT; it++) {
+            const int b = j + it * TPL;
+            if (IT * TPL == NB || b < NB) {
+#pragma unroll
+                for (int r = 0; r < R; r++) v[it][r] = lds[line * LD + b + r * NB];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int it = 0; it < IT; it++) {
+            const int b = j + it * TPL;
+            if (IT * TPL == NB || b < NB) {
+#pragma unroll
+                for (int r = 1; r < R; r++) v[it][r] = twmul(v[it][r], tw[TWO + b * (R - 1) + (r - 1)]);
+                bfly<T, R>::run(v[it]);
+#pragma unroll
+                for (int s = 0; s < R; s++) v[it][s] = conj(twmul(v[it][s], bh[b + s * NB]));
+                bfly<T, R>::run(v[it]);
+#pragma unroll
+                for (int s = 0; s < R; s++) lds[line * LD + b * R + s] = v[it][s];
+            }
+        }
+    }
+
+    // passes p .. p_end - 1 in place in LDS, a barrier after each
+    template <int p, int p_end, int LD>
+    static __device__ __forceinline__ void inner(const tw_t* __restrict__ tw, cx<T>* lds) {
+        if constexpr (p < p_end) {
+            auto ld = [&](int line, int n) { return lds[line * LD + n]; };
+            auto st = [&](int line, int n, cx<T> y) { lds[line * LD + n] = y; };
+            run<p, false, true>(tw, ld, st);
+            __syncthreads();
+            inner<p + 1, p_end, LD>(tw, lds);
+        }
+    }
+};
+}  // namespace dtfft
+
+// S: the schedule of M; SR: its radices in reverse (CHIRP only, with the table twr).
+// IN_COLS / OUT_COLS: lines adjacent in memory on that side, so threads run across lines.
+template <typename T, class S, class SR, int TPL, int LPB, int PAD, int KIND, bool CHIRP, bool IN_COLS, bool OUT_COLS>
 __global__ void __launch_bounds__(TPL * LPB)
 fft_any_kernel(const void* __restrict__ in_, void* __restrict__ out_,
-               const typename tw_of<T>::type* __restrict__ tw,
-               const typename tw_of<T>::type* __restrict__ chirp,
-               const typename tw_of<T>::type* __restrict__ bh, dtfft::lines_desc d, int inv, int n) {
-    typedef dtfft::fft_tile<T, S, TPL, LPB, false, false, PAD> F;
-    constexpr int M = S::N;
-    __shared__ cx<T> lds[F::LDS_ELEMS];
+               const typename tw_of<T>::type* __restrict__ tw_,
+               const typename tw_of<T>::type* __restrict__ twr_,
+               const typename tw_of<T>::type* __restrict__ chirp_,
+               const typename tw_of<T>::type* __restrict__ bh_, dtfft::lines_desc d, int inv, int n) {
+    typedef dtfft::any_passes<T, S, TPL, LPB> F;
+    typedef dtfft::any_passes<T, SR, TPL, LPB> B;
+    constexpr int NP = S::NP, LD = S::N + PAD;
+    __shared__ cx<T> lds[LPB * LD];
     const bool iv = KIND == 2 ? true : (KIND == 1 ? false : inv != 0);
     const int nout = KIND == 1 ? n / 2 + 1 : n;
-    // thread mapping along the lines where lines are adjacent in memory, else along them
-    const bool lfast_in = d.in_ls == 1 && d.in_ns != 1;
-    const bool lfast_out = d.out_ls == 1 && d.out_ns != 1;
     for (i64 t = blockIdx.x; t < d.ntiles; t += gridDim.x) {
-        i64 l0, ibase, obase;
-        F::tile_bases(d, t, l0, ibase, obase);
-        for (int e = threadIdx.x; e < LPB * M; e += F::NT) {
-            int line, m;
-            if (lfast_in) { line = e % LPB; m = e / LPB; }
-            else { line = e / M; m = e % M; }
+        const i64 l0 = t % d.ntl * LPB, bt = t / d.ntl;
+        const i64 ibase = l0 * d.in_ls + bt * d.in_bs, obase = l0 * d.out_ls + bt * d.out_bs;
+        const int lines = (int)(d.nl - l0 < LPB ? d.nl - l0 : LPB);
+        const auto* tw = fresh(tw_);
+        const auto* twr = fresh(twr_);
+        const auto* chirp = fresh(chirp_);
+        const auto* bh = fresh(bh_);
+        auto gload = [&](int line, int m) {
             cx<T> v = mk((T)0, (T)0);
-            if (m < n && l0 + line < d.nl) {
+            if (m < n && line < lines) {
                 const i64 lb = ibase + (i64)line * d.in_ls;
                 if constexpr (KIND == 0) {
                     v = ((const cx<T>*)in_)[lb + (i64)m * d.in_ns];
@@ -56,41 +162,42 @@ fft_any_kernel(const void* __restrict__ in_, void* __restrict__ out_,
                     v = mk(((const T*)in_)[lb + (i64)m * d.in_ns], (T)0);
                 } else {
                     const cx<T>* in = (const cx<T>*)in_;
-                    const int h = n / 2;
-                    if (m <= h) v = in[lb + (i64)m * d.in_ns];
+                    if (m <= n / 2) v = in[lb + (i64)m * d.in_ns];
                     else v = conj(in[lb + (i64)(n - m) * d.in_ns]);
                     if (m == 0 || 2 * m == n) v.y = (T)0;
                     v = conj(v);  // backward = conj(forward(conj))
                 }
                 if constexpr (CHIRP) v = twmul(v, chirp[m]);
             }
-            lds[line * F::LD + F::lidx(m)] = v;
-        }
-        __syncthreads();
-        F::template passes<0, false, false>(nullptr, nullptr, tw, lds, 0, 0, d, l0, false);
-        __syncthreads();
-        if constexpr (CHIRP) {
-            // pointwise product with DFT_M(b) / M, conjugated for the inverse transform
-            for (int e = threadIdx.x; e < LPB * M; e += F::NT) {
-                const int line = e / M, k = e % M;
-                cx<T>* r = &lds[line * F::LD + F::lidx(k)];
-                *r = conj(twmul(*r, bh[k]));
+            return v;
+        };
+        auto gstore = [&](int line, int k, cx<T> y) {
+            if (k < nout && line < lines) {
+                if constexpr (CHIRP) y = twmul(conj(y), chirp[k]);
+                const i64 o = obase + (i64)line * d.out_ls + (i64)k * d.out_ns;
+                if constexpr (KIND == 0) ((cx<T>*)out_)[o] = iv ? conj(y) : y;
+                else if constexpr (KIND == 1) ((cx<T>*)out_)[o] = y;
+                else ((T*)out_)[o] = y.x;  // real part; the conjugation leaves it unchanged
             }
+        };
+        auto sload = [&](int line, int m) { return lds[line * LD + m]; };
+        auto sstore = [&](int line, int m, cx<T> y) { lds[line * LD + m] = y; };
+        if constexpr (NP == 0) {  // one point
+            for (int line = threadIdx.x; line < LPB; line += F::NT) gstore(line, 0, gload(line, 0));
+        } else if constexpr (NP == 1) {  // direct only: a whole line in the registers of a thread
+            F::template run<0, IN_COLS, true>(tw, gload, gstore);
+        } else {
+            F::template run<0, IN_COLS, false>(tw, gload, sstore);
             __syncthreads();
-            F::template passes<0, false, false>(nullptr, nullptr, tw, lds, 0, 0, d, l0, false);
-            __syncthreads();
-        }
-        for (int e = threadIdx.x; e < LPB * nout; e += F::NT) {
-            int line, k;
-            if (lfast_out) { line = e % LPB; k = e / LPB; }
-            else { line = e / nout; k = e % nout; }
-            if (l0 + line >= d.nl) continue;
-            cx<T> y = lds[line * F::LD + F::lidx(k)];
-            if constexpr (CHIRP) y = twmul(conj(y), chirp[k]);
-            const i64 o = obase + (i64)line * d.out_ls + (i64)k * d.out_ns;
-            if constexpr (KIND == 0) ((cx<T>*)out_)[o] = iv ? conj(y) : y;
-            else if constexpr (KIND == 1) ((cx<T>*)out_)[o] = y;
-            else ((T*)out_)[o] = y.x;  // real part; the conjugation leaves it unchanged
+            F::template inner<1, NP - 1, LD>(tw, lds);
+            if constexpr (CHIRP) {
+                F::template turn<LD>(tw, bh, lds);
+                __syncthreads();
+                B::template inner<1, NP - 1, LD>(twr, lds);
+                B::template run<NP - 1, OUT_COLS, false>(twr, sload, gstore);
+            } else {
+                F::template run<NP - 1, OUT_COLS, false>(tw, sload, gstore);
+            }
         }
         __syncthreads();
     }

@@ -69,4 +69,13 @@ __device__ __forceinline__ void store_nt(cx<double>* p, cx<double> v) {
     __builtin_nontemporal_store(*(const u64x2*)&v, (u64x2*)p);
 }
 
+// p, as a value that the compiler takes for a new one: reads through it are not moved out of the
+// loop over tiles.  Most blocks run one tile, and the table entries of every pass would sit in
+// registers through all of it (fft_any_kernel, 640 = 8 10 8 in FP32: 216 VGPRs, 124 with this).
+template <typename P> __device__ __forceinline__ const P* fresh(const P* p) {
+    unsigned z;
+    asm volatile("s_mov_b32 %0, 0" : "=s"(z));
+    return p + z;
+}
+
 #endif

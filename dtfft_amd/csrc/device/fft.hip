@@ -1,7 +1,7 @@
 // Batched 1D C2C Stockham FFT kernels (register butterflies, LDS exchange).
 //
 // One thread block transforms LPB lines of length N.  The N-point transform
-// is a sequence of radix-R passes (R in 2,3,4,5,7,8,11,13,16); pass p with span
+// is a sequence of radix-R passes (R from 2 to 16, primes up to 61); pass p with span
 // L = R_0*...*R_{p-1} reads x[j + r*N/R], multiplies by w_{L*R}^{r*(j%L)},
 // runs an R-point DFT in registers and writes y[(j - j%L)*R + j%L + s*L].
 // The first pass reads global memory directly and the last pass writes it
@@ -178,6 +178,121 @@ template <typename T> struct bfly<T, 7> : bfly_prime<T, 7> {};
 template <typename T> struct bfly<T, 11> : bfly_prime<T, 11> {};
 template <typename T> struct bfly<T, 13> : bfly_prime<T, 13> {};
 
+// Composite radices.  A pass costs one exchange of the line through LDS and one twiddle product
+// per element whatever its radix, so 210 = 14 15 takes two passes where 2 3 5 7 takes four.
+// Coprime factors A B (Good-Thomas): with n = B n1 + A n2 mod A B and k known by its residues,
+// w^{nk} = w_A^{n1 (k mod A)} w_B^{n2 (k mod B)} -- an A x B transform without twiddles.
+template <typename T, int A, int B> struct bfly_coprime {
+    static __device__ __forceinline__ void run(cx<T>* v) {
+        cx<T> u[A][B];
+#pragma unroll
+        for (int n2 = 0; n2 < B; n2++) {
+            cx<T> t[A];
+#pragma unroll
+            for (int n1 = 0; n1 < A; n1++) t[n1] = v[(B * n1 + A * n2) % (A * B)];
+            bfly<T, A>::run(t);
+#pragma unroll
+            for (int k1 = 0; k1 < A; k1++) u[k1][n2] = t[k1];
+        }
+#pragma unroll
+        for (int k1 = 0; k1 < A; k1++) bfly<T, B>::run(u[k1]);
+#pragma unroll
+        for (int k = 0; k < A * B; k++) v[k] = u[k % A][k % B];
+    }
+};
+template <typename T> struct bfly<T, 6> : bfly_coprime<T, 2, 3> {};
+template <typename T> struct bfly<T, 10> : bfly_coprime<T, 2, 5> {};
+template <typename T> struct bfly<T, 12> : bfly_coprime<T, 4, 3> {};
+template <typename T> struct bfly<T, 14> : bfly_coprime<T, 2, 7> {};
+template <typename T> struct bfly<T, 15> : bfly_coprime<T, 3, 5> {};
+
+template <typename T> struct bfly<T, 9> {
+    static __device__ __forceinline__ void run(cx<T>* v) {
+        // 9 = 3 x 3, twiddles w9^(n1 k0) in between, as radix 16
+        const T c1 = (T)0.766044443118978, s1 = (T)0.6427876096865393;   // w9^1 = c1 - i s1
+        const T c2 = (T)0.17364817766693036, s2 = (T)0.984807753012208;  // w9^2
+        const T c4 = (T)-0.9396926207859084, s4 = (T)0.3420201433256687; // w9^4
+        cx<T> u[3][3];
+#pragma unroll
+        for (int n1 = 0; n1 < 3; n1++) {
+            cx<T> t[3] = {v[n1], v[n1 + 3], v[n1 + 6]};
+            bfly<T, 3>::run(t);
+#pragma unroll
+            for (int k0 = 0; k0 < 3; k0++) u[k0][n1] = t[k0];
+        }
+        u[1][1] = cmulc(u[1][1], c1, -s1);
+        u[1][2] = cmulc(u[1][2], c2, -s2);
+        u[2][1] = cmulc(u[2][1], c2, -s2);
+        u[2][2] = cmulc(u[2][2], c4, -s4);
+#pragma unroll
+        for (int k0 = 0; k0 < 3; k0++) {
+            bfly<T, 3>::run(u[k0]);
+#pragma unroll
+            for (int k1 = 0; k1 < 3; k1++) v[k0 + 3 * k1] = u[k0][k1];
+        }
+    }
+};
+
+// cos and sin of 2 pi k / P, k <= P / 2, at compile time: the angle is folded into the first
+// octant in integers and the Taylor series of sin and cos summed there (12 terms, below the
+// last place of a double at pi / 4).
+template <int P> struct circle {
+    double c[P / 2 + 1], s[P / 2 + 1];
+    static constexpr double series(double x, bool odd) {
+        const double x2 = x * x;
+        double r = 1.0;
+        for (int i = 12; i >= 1; i--) r = 1.0 - r * x2 / (odd ? (2.0 * i) * (2.0 * i + 1.0) : (2.0 * i - 1.0) * (2.0 * i));
+        return odd ? x * r : r;
+    }
+    constexpr circle() : c(), s() {
+        const double pi = 3.14159265358979323846;
+        for (int k = 0; k <= P / 2; k++) {
+            if (8 * k <= P) {
+                const double x = 2.0 * pi * k / P;
+                c[k] = series(x, false); s[k] = series(x, true);
+            } else if (8 * k <= 3 * P) {  // around pi / 2: x = angle - pi / 2
+                const double x = pi * (4 * k - P) / (2.0 * P);
+                c[k] = -series(x, true); s[k] = series(x, false);
+            } else {  // x = pi - angle
+                const double x = pi * (P - 2 * k) / (double)P;
+                c[k] = -series(x, false); s[k] = series(x, true);
+            }
+        }
+    }
+};
+
+// Primes above 13 as radices of their own: (R - 1)^2 multiply-adds per butterfly, in registers,
+// where Bluestein's transform of the line would run two transforms of twice its length.  Outputs
+// go to emit(s, y_s) as they are done, so only the inputs are held.
+template <typename T, int R, class Emit>
+__device__ __forceinline__ void bfly_large(cx<T>* v, const Emit& emit) {
+    static_assert(R > 16 && R % 2 == 1, "a prime");
+    constexpr int H = (R - 1) / 2;
+    constexpr circle<R> w;
+    cx<T> y0 = v[0];
+#pragma unroll
+    for (int r = 1; r <= H; r++) {  // v[r] <- x_r + x_{R-r}, v[R-r] <- x_r - x_{R-r}
+        const cx<T> a = v[r], b = v[R - r];
+        v[r] = a + b;
+        v[R - r] = a - b;
+        y0 = y0 + v[r];
+    }
+    emit(0, y0);
+#pragma unroll
+    for (int s = 1; s <= H; s++) {
+        cx<T> a = v[0], b = mk((T)0, (T)0);
+#pragma unroll
+        for (int r = 1; r <= H; r++) {
+            const int q = (r * s) % R;
+            const int qq = q <= H ? q : R - q;
+            a = a + scale(v[r], (T)w.c[qq]);
+            b = b + scale(v[R - r], (T)(q <= H ? w.s[qq] : -w.s[qq]));
+        }
+        emit(s, mk(a.x + b.y, a.y - b.x));
+        emit(R - s, mk(a.x - b.y, a.y + b.x));
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Radix schedule (compile time).
 // ---------------------------------------------------------------------------
@@ -226,7 +341,12 @@ struct lines_desc {
 // the per-peer chunks of a receive buffer, so that unpack and FFT are one pass.
 // OSEG > 0 writes the FFT axis in segments of OSEG elements that lie out_seg_stride apart:
 // the chunk-blocked layout that a following column-in pass reads as contiguous tiles.
-template <typename T, class S, int TPL, int LPB, bool IN_COLS, bool OUT_COLS, int PAD, int SEG = 0, int OSEG = 0>
+// STAGED: the tile goes through LDS on its way in and out.  Without it, thread j of a line reads
+// elements j + r N / R and writes j + s L, TPL neighbours at a time.  Where TPL is large, the way
+// through LDS costs more than it gives (384-point FP32 rows 82 against 152 us per 256 MB); for the
+// few threads of a schedule like 37 2 it gives: 74 points 173 against 294 us.
+template <typename T, class S, int TPL, int LPB, bool IN_COLS, bool OUT_COLS, int PAD, int SEG = 0, int OSEG = 0,
+          bool STAGED = false>
 struct fft_tile {
     static __device__ __forceinline__ i64 in_elem(int n, const lines_desc& d) {
         if constexpr (SEG > 0) return (i64)(n / SEG) * d.in_seg_stride + (i64)(n % SEG) * d.in_ns;
@@ -311,14 +431,11 @@ struct fft_tile {
                     for (int r = 1; r < R; r++)
                         v[it][r] = twmul(v[it][r], tw[TWO + k * (R - 1) + (r - 1)]);
                 }
-                bfly<T, R>::run(v[it]);
                 const int base = (b - k) * R + k;
-#pragma unroll
-                for (int s = 0; s < R; s++) {
+                auto put = [&](int s, cx<T> y) {
                     const int n = base + s * L;
                     if (DST_G) {
                         if (lv) {
-                            cx<T> y = v[it][s];
                             cx<T>* o = &gout[obase + (i64)line * d.out_ls + out_elem(n, d)];
                             // rows in and rows out: non-temporal stores (measured faster on MI355X
                             // for the row passes, slower for column-in and column-out passes)
@@ -331,8 +448,15 @@ struct fft_tile {
                         // share one 16-element group
                         const int q = (L % 16 == 0) ? lidx(base) + s * lspan(L)
                                       : (L == 1 && 16 % R == 0) ? lidx(base) + s : lidx(n);
-                        lds[line * LD + q] = v[it][s];
+                        lds[line * LD + q] = y;
                     }
+                };
+                if constexpr (R > 16) {
+                    bfly_large<T, R>(v[it], put);
+                } else {
+                    bfly<T, R>::run(v[it]);
+#pragma unroll
+                    for (int s = 0; s < R; s++) put(s, v[it][s]);
                 }
             }
         }
@@ -362,17 +486,17 @@ struct fft_tile {
             constexpr bool first = (p == 0);
             constexpr bool last = (p == NP - 1);
             if constexpr (first && FIRST_G && last) {
-                // single pass from global: stage the input through LDS so that in-place use
-                // is safe and the read and write mappings may differ
-                for (int e = threadIdx.x; e < LPB * N && (int)threadIdx.x < NT; e += NT) {
-                    int line, n;
-                    if (IN_COLS) { line = e % LPB; n = e / LPB; } else { line = e / N; n = e % N; }
-                    cx<T> x = mk((T)0, (T)0);
-                    if (l0 + line < d.nl) x = gin[ibase + (i64)line * d.in_ls + in_elem(n, d)];
-                    lds[line * LD + lidx(n)] = inv ? conj(x) : x;
-                }
+                // single pass from global: the tile goes through LDS, so that in-place use is
+                // safe and the global accesses are whole rows whatever the thread mapping (one
+                // thread holds a line; 13-point FP32 rows, 256 MB: 1186 us stored from there,
+                // 113 us through LDS)
+                stage_in(gin, lds, ibase, d, l0, inv);
                 __syncthreads();
-                pass<p, false, LAST_G, OUT_COLS>(gin, gout, tw, lds, ibase, obase, d, l0, inv);
+                pass<p, false, false, false>(gin, gout, tw, lds, ibase, obase, d, l0, inv);
+                if constexpr (LAST_G) {
+                    __syncthreads();
+                    stage_out(gout, lds, obase, d, l0, inv);
+                }
             } else if constexpr (first && FIRST_G) {
                 pass<p, true, false, IN_COLS>(gin, gout, tw, lds, ibase, obase, d, l0, inv);
             } else if constexpr (first) {
@@ -398,6 +522,34 @@ struct fft_tile {
         obase = l0 * d.out_ls + b * d.out_bs;
     }
 
+    // The tile between global memory and LDS, neighbouring threads on neighbouring elements of
+    // a line (rows) or on neighbouring lines (columns) over the whole block.
+    static __device__ __forceinline__ void stage_in(const cx<T>* __restrict__ gin, cx<T>* lds, i64 ibase,
+                                                    const lines_desc& d, i64 l0, bool inv) {
+        constexpr int IT = (LPB * N + NT - 1) / NT;
+#pragma unroll 8
+        for (int i = 0; i < IT; i++) {
+            const int e = (int)threadIdx.x + i * NT;
+            if ((int)threadIdx.x >= NT || e >= LPB * N) break;
+            const int line = IN_COLS ? e % LPB : e / N, n = IN_COLS ? e / LPB : e % N;
+            cx<T> x = mk((T)0, (T)0);
+            if (l0 + line < d.nl) x = gin[ibase + (i64)line * d.in_ls + in_elem(n, d)];
+            lds[line * LD + lidx(n)] = inv ? conj(x) : x;
+        }
+    }
+    static __device__ __forceinline__ void stage_out(cx<T>* __restrict__ gout, const cx<T>* lds, i64 obase,
+                                                     const lines_desc& d, i64 l0, bool inv) {
+        constexpr int IT = (LPB * N + NT - 1) / NT;
+#pragma unroll 8
+        for (int i = 0; i < IT; i++) {
+            const int e = (int)threadIdx.x + i * NT;
+            if ((int)threadIdx.x >= NT || e >= LPB * N) break;
+            const int line = OUT_COLS ? e % LPB : e / N, n = OUT_COLS ? e / LPB : e % N;
+            const cx<T> y = lds[line * LD + lidx(n)];
+            if (l0 + line < d.nl) gout[obase + (i64)line * d.out_ls + out_elem(n, d)] = inv ? conj(y) : y;
+        }
+    }
+
     static __device__ __forceinline__ void run(const cx<T>* __restrict__ gin, cx<T>* __restrict__ gout,
                                                const tw_t* __restrict__ tw, cx<T>* lds,
                                                const lines_desc& d, i64 tile, bool inv) {
@@ -405,6 +557,12 @@ struct fft_tile {
         tile_bases(d, tile, l0, ibase, obase);
         if constexpr (NP == 0) {
             return;
+        } else if constexpr (STAGED) {
+            stage_in(gin, lds, ibase, d, l0, inv);
+            __syncthreads();
+            passes<0, false, false>(gin, gout, tw, lds, ibase, obase, d, l0, inv);
+            __syncthreads();
+            stage_out(gout, lds, obase, d, l0, inv);
         } else {
             passes<0, true, true>(gin, gout, tw, lds, ibase, obase, d, l0, inv);
         }
@@ -435,11 +593,11 @@ __device__ __forceinline__ i64 xcd_tile(i64 slot, i64 G) {
 }  // namespace dtfft
 
 template <typename T, class S, int TPL, int LPB, bool IN_COLS, bool OUT_COLS, int PAD, int SEG = 0, bool TWL = false,
-          int OSEG = 0>
+          int OSEG = 0, bool STAGED = false>
 __global__ void __launch_bounds__(TPL * LPB)
 fft_c2c_kernel(const cx<T>* __restrict__ in, cx<T>* __restrict__ out,
                const typename tw_of<T>::type* __restrict__ tw, dtfft::lines_desc d, int inv) {
-    typedef dtfft::fft_tile<T, S, TPL, LPB, IN_COLS, OUT_COLS, PAD, SEG, OSEG> F;
+    typedef dtfft::fft_tile<T, S, TPL, LPB, IN_COLS, OUT_COLS, PAD, SEG, OSEG, STAGED> F;
     typedef typename tw_of<T>::type tw_t;
     __shared__ cx<T> lds[F::LDS_ELEMS];
     const tw_t* twp = tw;

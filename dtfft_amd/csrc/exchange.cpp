@@ -53,7 +53,7 @@ int32_t dtfft_hip_unpack_fft_create(int32_t ndims, const int32_t* dims, const in
     const bool dbl = precision == DTFFT_HIP_DOUBLE;
     std::vector<int> rad;
     if (!factorize((int)nx, rad)) return DTFFT_HIP_ERROR_UNSUPPORTED_SIZE;
-    fft_config c = default_fft_config((int)nx, dbl, false, false, false);
+    fft_config c = default_fft_config((int)nx, dbl, false, false, ny * nz, ny * nz);
     c.seg = (int)seg;
     // line (y, z) = l: input base l * seg (inside chunk 0) + din_0, output l * nx
     lines_desc d = make_lines(ny * nz, 1, seg, 0, 1, nx, 0, 1, c.lpb);

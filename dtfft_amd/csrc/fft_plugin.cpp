@@ -19,8 +19,14 @@
 
 namespace dtfft_hip {
 
+// Primes above 13 that the kernels have as radices of their own (bfly in device/fft.hip).
+static const int kLargePrimes[] = {17, 19, 23, 29, 31, 37, 41, 43, 47, 53, 59, 61};
+static bool large_prime(int r) {
+    return std::find(std::begin(kLargePrimes), std::end(kLargePrimes), r) != std::end(kLargePrimes);
+}
+
 // ---- schedules ----------------------------------------------------------------------
-bool factorize(int n, std::vector<int>& radices) {
+bool prime_schedule(int n, std::vector<int>& radices) {
     radices.clear();
     if (n < 1) return false;
     if (n == 1) { radices.push_back(1); return true; }
@@ -41,13 +47,94 @@ bool factorize(int n, std::vector<int>& radices) {
     return true;
 }
 
+// Share of thread-rounds that do work when a line's passes run on tpl threads, inverted: 1 when
+// every pass fills its rounds of butterflies, 2 when half of the threads wait.
+static double idle_factor(const std::vector<int>& radices, int n, int tpl) {
+    double sum = 0;
+    for (int r : radices) sum += (double)((n / r + tpl - 1) / tpl) * tpl * r;
+    return sum / ((double)n * (double)radices.size());
+}
+
+// Threads per line with the least idle rounds: the butterflies of one of the passes.
+static int best_tpl(const std::vector<int>& radices, int n) {
+    int best = 1;
+    double bf = 1e30;
+    for (int r : radices) {
+        const int t = n / r;
+        const double f = idle_factor(radices, n, t);
+        if (f < bf - 1e-9 || (f < bf + 1e-9 && t > best)) { bf = f; best = t; }
+    }
+    return best;
+}
+
+// The radix schedule of n: fewest passes of radices up to 16 -- but two for 6 to 16, where one
+// thread would hold a whole line (16 = 4 4 on four threads 78 us per 256 MB of FP32 rows, 135 us
+// as one radix 16) -- then the least idle rounds and the smallest radix.
+bool factorize(int n, std::vector<int>& radices) {
+    if (!prime_schedule(n, radices)) return false;  // a prime above 13
+    if (n == 1) return true;
+    static std::mutex mu;
+    static std::map<int, std::vector<int>> known;  // plans ask for a few lengths many times
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        auto it = known.find(n);
+        if (it != known.end()) { radices = it->second; return true; }
+    }
+    std::vector<int> cur, best;
+    double cost = 1e30;
+    std::function<void(int, int)> rec = [&](int m, int hi) {
+        if (m == 1) {
+            double f = 100.0 * (double)cur.size() + 16.0 * idle_factor(cur, n, best_tpl(cur, n)) + cur[0];
+            for (int r : cur) f += 0.01 * r;
+            if (n >= 6 && cur.size() == 1) f += 200.0;
+            if (f < cost) { cost = f; best = cur; }
+            return;
+        }
+        if (cur.size() >= 10 || (!best.empty() && cur.size() >= std::max<size_t>(2, best.size()))) return;
+        for (int r = std::min(hi, 16); r >= 2; r--)
+            if (m % r == 0) {
+                cur.push_back(r);
+                rec(m / r, r);
+                cur.pop_back();
+            }
+    };
+    rec(n, 16);
+    if (!best.empty()) radices = best;
+    std::lock_guard<std::mutex> lk(mu);
+    known[n] = radices;
+    return true;
+}
+
+// Schedules of lengths with prime factors above 13 that have radices of their own, those first:
+// the first pass needs no twiddles, 36 of them per butterfly of 37.  Only lengths that the
+// Bluestein form would take (its work line fits the LDS) and only up to max_prime.
+bool large_schedule(int n, bool dbl, int max_prime, std::vector<int>& radices) {
+    radices.clear();
+    if (2 * (int64_t)n - 1 > (int64_t)(160 * 1024 / (dbl ? 16 : 8))) return false;
+    int m = n;
+    std::vector<int> rest;
+    for (int p : kLargePrimes)
+        while (p <= max_prime && m % p == 0) { radices.insert(radices.begin(), p); m /= p; }
+    if (radices.empty() || !factorize(m, rest)) return false;
+    if (m <= 16) rest = {m};
+    if (m > 1) radices.insert(radices.end(), rest.begin(), rest.end());
+    return radices.size() <= 10;
+}
+
 std::string fft_config::expr() const {
     if (any) {
-        std::string s = std::string("fft_any_kernel<") + (dbl ? "double" : "float") + ", dtfft::sched<" +
-                        std::to_string(n);
-        for (int r : radices) s += ", " + std::to_string(r);
-        return s + ">, " + std::to_string(tpl) + ", " + std::to_string(lpb) + ", " + std::to_string(pad) + ", " +
-               std::to_string(kind) + (chirp ? ", true>" : ", false>");
+        // the schedule, and its radices in reverse for the second transform of Bluestein's form
+        std::string s = std::string("fft_any_kernel<") + (dbl ? "double" : "float");
+        const std::vector<int> rev(radices.rbegin(), radices.rend());
+        for (const auto* r : {&radices, &rev}) {
+            s += ", dtfft::sched<" + std::to_string(n);
+            for (int x : *r) s += ", " + std::to_string(x);
+            s += ">";
+        }
+        s += ", " + std::to_string(tpl) + ", " + std::to_string(lpb) + ", " + std::to_string(pad) + ", " +
+             std::to_string(kind);
+        for (bool b : {chirp, in_cols, out_cols}) s += b ? ", true" : ", false";
+        return s + ">";
     }
     if (dma && kind == 2) {
         std::string s = std::string(dma == 1 ? "fft_c2r_dma2_kernel<" : "fft_c2r_dma_kernel<") +
@@ -71,9 +158,10 @@ std::string fft_config::expr() const {
     s += ">, " + std::to_string(tpl) + ", " + std::to_string(lpb) + ", ";
     if (kind == 0) s += std::string(in_cols ? "true" : "false") + ", " + (out_cols ? "true" : "false") + ", ";
     s += std::to_string(pad);
-    if (kind == 0 && (seg > 0 || twl || oseg > 0)) s += ", " + std::to_string(seg);
-    if (kind == 0 && (twl || oseg > 0)) s += twl ? ", true" : ", false";
-    if (kind == 0 && oseg > 0) s += ", " + std::to_string(oseg);
+    if (kind == 0 && (seg > 0 || twl || oseg > 0 || staged)) s += ", " + std::to_string(seg);
+    if (kind == 0 && (twl || oseg > 0 || staged)) s += twl ? ", true" : ", false";
+    if (kind == 0 && (oseg > 0 || staged)) s += ", " + std::to_string(oseg);
+    if (kind == 0 && staged) s += ", true";
     if (kind == 1 && oseg > 0) s += ", " + std::to_string(oseg);
     if (kind == 2 && (in_cols || twl)) s += in_cols ? ", true" : ", false";
     if (kind == 2 && twl) s += ", true";
@@ -183,39 +271,86 @@ void apply_twl(fft_config& c, const lines_desc& d, int mode) {
     if (!valid(c)) c.twl = 0;  // tile + tables over the LDS budget: global twiddles
 }
 
-fft_config default_fft_config(int n, bool dbl, bool in_cols, bool out_cols, bool inplace) {
-    (void)inplace;
+// Schedule and threads per line of n for `points` elements per thread.  Up to two passes: the
+// largest radix first and n / rmin threads, one butterfly each in the second pass (84 = 12 7 on
+// 12 threads 216 us per GiB of FP32 rows, on 7 threads 483; column tiles 192 against 238).  More
+// passes: of the schedules of fewest passes, the one with the least idle rounds on the smallest
+// power of two (16 at least) of threads that leaves at most `points` elements to each, radices
+// descending: whole waves then hold whole lines (384 FP32 columns: 12 8 4 on 16 threads 226 us,
+// 8 8 6 on 48 285 us).
+void pick_schedule(int n, int points, std::vector<int>& radices, int& tpl) {
+    if (!factorize(n, radices)) return;
+    tpl = 1;
+    if (radices.size() == 1) return;
+    if (radices.size() == 2) { tpl = n / radices[1]; return; }
+    tpl = 16;
+    while (n > tpl * points) tpl *= 2;
+    const size_t np = radices.size();
+    std::vector<int> cur;
+    double best = 1e30;
+    std::function<void(int, int)> rec = [&](int m, int hi) {
+        if (m == 1) {
+            double f = idle_factor(cur, n, tpl);
+            for (int r : cur) f += 1e-4 * r;  // equal otherwise: the smaller radices
+            if (cur.size() == np && f < best) { best = f; radices = cur; }
+            return;
+        }
+        if (cur.size() >= np) return;
+        for (int r = std::min(hi, 16); r >= 2; r--)
+            if (m % r == 0) {
+                cur.push_back(r);
+                rec(m / r, r);
+                cur.pop_back();
+            }
+    };
+    rec(n, 16);
+}
+
+fft_config default_fft_config(int n, bool dbl, bool in_cols, bool out_cols, int64_t lines, int64_t nl) {
     fft_config c;
     c.n = n; c.dbl = dbl; c.in_cols = in_cols; c.out_cols = out_cols;
-    factorize(n, c.radices);
-    int rmax = *std::max_element(c.radices.begin(), c.radices.end());
-    c.tpl = std::max(1, n / rmax);
-    if (in_cols || out_cols) {
-        // Columns: 16 lines per tile (128-byte rows in FP32).  FP64 at n >= 256 takes 16
-        // lines too (256-byte rows) with two butterflies per thread, which measured faster
-        // on MI355X (512^3: 825 us per pass against 845 with 8 lines).
-        c.pad = 1;
-        c.lpb = dbl ? 8 : 16;
-        if (dbl && n >= 256) {
-            c.lpb = 16;
-            c.tpl = std::max(1, c.tpl / 2);
-        }
-        while (c.tpl * c.lpb > 1024 && c.tpl > 1) c.tpl = (c.tpl + 1) / 2;
-        while (!valid(c) && c.lpb > 1) c.lpb /= 2;
+    const bool cols = in_cols || out_cols;
+    const int es = elem_bytes(dbl);
+    // Launches that would not give every CU two tiles are bound by latency, not by HBM: one
+    // butterfly per thread (8 elements) and the smallest tiles.  A 512-point FP32 row pass of
+    // 0.7 MB takes 4.0 us with one line per block, 4.7 us with four; column passes 5.6 us with 8
+    // lines, 7.5 us with 16.
+    const int wide = cols ? (dbl ? 8 : 16) : 4;
+    const bool few = lines > 0 && lines < (int64_t)wide * 512;
+    if (large_schedule(n, dbl, kMaxPrime(dbl), c.radices)) {
+        // One butterfly of the prime per thread and at most 24 points in the other passes (444 =
+        // 37 12 on 12 threads: four butterflies of 12, 332 VGPRs); rows prefer one butterfly of
+        // the last pass while those are few (136 = 17 8 FP32: 17 threads 86 us per 256 MB, 8
+        // threads 289; 333 = 37 9: 37 threads 219, 14 threads 209).
+        const int last = n / c.radices.back();
+        c.tpl = std::max(n / c.radices[0], (n + 23) / 24);
+        if (!cols && c.radices.size() == 2 && last <= 31) c.tpl = last;
+        c.staged = !cols && c.radices.size() == 2 && c.radices[1] <= 4;
     } else {
-        // Rows: small blocks (about 128 threads in FP32, 64 in FP64, 256 once a line takes 64
-        // threads or more), several resident per CU so that one block's loads overlap
-        // another's passes; at n = 512..1024 (FP32) and 512 (FP64) two butterflies per thread
-        // and pass measured faster on MI355X (512 FP32: 5.6 TB/s against 5.2 with one; 512
-        // FP64: 731 us per pass with 2 lines per block against 763 with 4).
-        c.pad = 0;
-        if ((!dbl && n >= 512 && n <= 1024) || (dbl && n == 512)) c.tpl = std::max(1, c.tpl / 2);
-        const int target = c.tpl >= 64 ? 256 : (dbl ? 64 : 128);
-        c.lpb = 1;
-        while (c.lpb * c.tpl < target) c.lpb *= 2;
-        while ((size_t)c.lpb * lds_line(n, c.pad) * elem_bytes(dbl) > 64 * 1024 && c.lpb > 1) c.lpb /= 2;
-        while (c.tpl * c.lpb > 1024 && c.tpl > 1) c.tpl = (c.tpl + 1) / 2;
+        // FP32 takes 24 elements per thread at most and FP64 16: the bytes in flight that hide
+        // the latency of HBM come from many loads per thread.
+        pick_schedule(n, few ? 8 : dbl ? 16 : 24, c.radices, c.tpl);
     }
+    if (cols) {
+        // FP32 16 lines per tile (128-byte pieces of rows), FP64 8; fewer where the tile leaves
+        // no room for three blocks per CU (512 points FP32: 8 lines 224 us, 16 lines 248 us; FP64
+        // at 384 points: 8 lines 195 us, 16 lines 237 us); more where a line has few threads
+        // (12 points FP32 on 4 threads: 64 lines 102 us, 32 lines 111 us per 256 MB).
+        c.pad = 1;
+        c.lpb = wide;
+        while (!dbl && c.lpb > 8 && (size_t)c.lpb * (size_t)n * (size_t)es > 52 * 1024) c.lpb /= 2;
+        while (c.lpb * 2 * c.tpl <= 128 && c.lpb < 64 && c.lpb < nl) c.lpb *= 2;
+        if (few) while (c.lpb * es > 64 && lines / c.lpb < 512) c.lpb /= 2;
+    } else {
+        // two waves per block (84 points FP32 on 12 threads: 10 lines 90 us, 5 lines 92 us per
+        // 256 MB; FP64 79 and 84 us)
+        c.pad = 0;
+        c.lpb = std::max(1, (c.tpl >= 128 ? 256 : 128) / c.tpl);
+        if (few) while (c.lpb > 1 && c.tpl * c.lpb >= 128 && lines / c.lpb < 512) c.lpb /= 2;
+    }
+    while (c.tpl * c.lpb > 1024 && c.lpb > 1) c.lpb /= 2;
+    while (c.tpl > 1024) c.tpl = (c.tpl + 1) / 2;
+    while (!valid(c) && c.lpb > 1) c.lpb /= 2;
     return c;
 }
 
@@ -230,7 +365,9 @@ std::vector<std::vector<int>> radix_schedules(int n, int max_count) {
     int a = 0, m = n;
     while (m % 2 == 0) { m /= 2; a++; }
     std::vector<int> odd;
-    for (int r : def)
+    std::vector<int> primes;
+    prime_schedule(n, primes);
+    for (int r : primes)
         if (r % 2 != 0 && r != 1) odd.push_back(r);
     std::vector<std::vector<int>> pow2;  // exponent lists, each in [1, 4]
     if (a == 0) pow2.push_back({});
@@ -269,9 +406,9 @@ std::vector<std::vector<int>> radix_schedules(int n, int max_count) {
     return out;
 }
 
-std::vector<fft_config> fft_candidates(int n, bool dbl, bool in_cols, bool out_cols, bool inplace) {
+std::vector<fft_config> fft_candidates(int n, bool dbl, bool in_cols, bool out_cols, int64_t lines, int64_t nl) {
     std::vector<fft_config> out;
-    fft_config base = default_fft_config(n, dbl, in_cols, out_cols, inplace);
+    fft_config base = default_fft_config(n, dbl, in_cols, out_cols, lines, nl);
     out.push_back(base);
     std::vector<int> lpbs;
     if (in_cols || out_cols) lpbs = {4, 8, 16, 32};
@@ -310,11 +447,15 @@ std::vector<fft_config> fft_candidates(int n, bool dbl, bool in_cols, bool out_c
     return out;
 }
 
-// Any-length kernel: the work line of m points sits whole in LDS.  Bluestein takes the
-// smallest m >= 2n - 1 whose primes are <= 7.  One butterfly of the
-// largest radix per thread and pass; lines per block grow to about 256 threads while the
-// tile stays within 64 KiB of LDS, so that several blocks share a CU.
-bool any_config(int kind, int n, bool dbl, bool direct, fft_config& c) {
+// Any-length kernel: the work line of m points sits whole in LDS.  Bluestein takes an
+// m >= 2n - 1, up to an eighth above it, that costs least: points times the passes (12 for the
+// trip through LDS, and the butterfly), and half of the threads that wait.  The largest radix goes to
+// the middle: the first and last pass hold chirps and global addresses, the turning pass (the last
+// radix) two tables.  One butterfly per thread in the first pass, blocks of about 160 threads.
+// Lines of 313 points, 128 MB in FP32: 640 = 10 8 8 or 8 10 8 on 80 threads 173-178 us, on 64
+// threads 196 us, 672 = 12 8 7 on 56 threads 202 us, the slowest of 90 shapes 399 us; 619 points:
+// 1280 = 10 16 8 on 128 threads 204 us, 8 16 10 on 160 threads 231 us, the slowest 712 us.
+bool any_config(int kind, int n, bool dbl, bool direct, bool cols, fft_config& c) {
     c = fft_config{};
     c.any = 1;
     c.kind = kind;
@@ -323,28 +464,38 @@ bool any_config(int kind, int n, bool dbl, bool direct, fft_config& c) {
     c.chirp = !direct;
     const int64_t es = elem_bytes(dbl);
     const int64_t mmax = (int64_t)(kMaxLds / (size_t)es);
-    int64_t m = direct ? n : 2 * (int64_t)n - 1;
-    for (;; m++) {
-        if (m > mmax) return false;
-        if (!factorize((int)m, c.radices)) {
-            if (direct) return false;
-            continue;
+    const int64_t lo = direct ? n : 2 * (int64_t)n - 1;
+    double best = 0;
+    for (int64_t m = lo; m <= mmax && (m == lo || !direct) && (best == 0 || m <= lo + lo / 8); m++) {
+        std::vector<int> r;
+        if (!factorize((int)m, r)) continue;
+        if (!direct) {
+            std::sort(r.begin(), r.end());
+            if (r.size() > 2) {  // smallest last, second largest first
+                std::rotate(r.begin(), r.begin() + 1, r.end());
+                std::swap(r.front(), r[r.size() - 3]);
+            }
         }
-        if (direct) break;
-        bool small = true;
-        for (int r : c.radices) small &= (r == 1 || r == 2 || r == 3 || r == 4 || r == 5 || r == 7 || r == 8 || r == 16);
-        if (small) break;
+        int tpl = direct ? best_tpl(r, (int)m) : (int)m / r[0];
+        while (tpl > 1024) tpl = (tpl + 1) / 2;
+        double cost = 0;
+        for (int x : r) cost += 12.0 + 0.3 * x + (x == 11 || x == 13 ? 8.0 : 0.0);
+        cost *= (double)m * std::sqrt(idle_factor(r, (int)m, tpl));
+        if (best != 0 && cost >= best) continue;
+        best = cost;
+        c.n = (int)m;
+        c.radices = r;
+        c.tpl = tpl;
     }
-    c.n = (int)m;
-    const int rmax = *std::max_element(c.radices.begin(), c.radices.end());
-    c.tpl = std::max<int>(1, (int)(m / rmax));
-    while (c.tpl > 1024) c.tpl = (c.tpl + 1) / 2;
-    c.lpb = 1;
-    c.pad = 0;
-    while (c.lpb * c.tpl < 256 && c.lpb * 2 * c.tpl <= 1024 &&
-           (size_t)(c.lpb * 2) * lds_line(c.n, 1) * (size_t)es <= 64 * 1024)
-        c.lpb *= 2;
-    if (c.lpb > 1) c.pad = 1;
+    if (best == 0) return false;
+    auto fits = [&](int l) {
+        return l * c.tpl <= 1024 && (size_t)l * lds_line(c.n, 1) * (size_t)es <= 64 * 1024;
+    };
+    c.lpb = std::max(1, (c.tpl <= 16 ? 256 : 160) / c.tpl);
+    while (c.lpb > 1 && !fits(c.lpb)) c.lpb /= 2;
+    // lines adjacent in memory: 64-byte pieces of them where the tile allows it
+    if (cols) while (c.lpb * es < 64 && fits(c.lpb * 2)) c.lpb *= 2;
+    c.pad = c.lpb > 1 ? 1 : 0;
     return valid(c);
 }
 
@@ -462,9 +613,15 @@ int32_t fft_stage::init(const fft_config& c, const lines_desc& desc) {
     d.ntl = (d.nl + c.lpb - 1) / c.lpb;
     d.ntiles = d.ntl * d.nb;
     if (c.any) {
-        TRY(rtc_get("anylen", c.expr(), &k));
+        // threads run across lines where the lines are adjacent in memory, else along them
+        cfg.in_cols = d.in_ls == 1 && d.in_ns != 1;
+        cfg.out_cols = d.out_ls == 1 && d.out_ns != 1;
+        TRY(rtc_get("anylen", cfg.expr(), &k));
         TRY(get_twiddles(c.n, c.radices, c.dbl, &tw));
-        if (c.chirp) TRY(get_bluestein(c.nlog, c.n, c.dbl, &chirp, &bh));
+        if (c.chirp) {
+            TRY(get_twiddles(c.n, {c.radices.rbegin(), c.radices.rend()}, c.dbl, &twr));
+            TRY(get_bluestein(c.nlog, c.n, c.dbl, &chirp, &bh));
+        }
         block = (unsigned)(c.tpl * c.lpb);
         grid = (unsigned)std::min<int64_t>(d.ntiles, 1 << 22);
         return DTFFT_HIP_SUCCESS;
@@ -523,11 +680,12 @@ int32_t fft_stage::run(const void* in, void* out, int sign, hipStream_t s) const
     if (d.ntiles == 0) return DTFFT_HIP_SUCCESS;
     if (cfg.any) {
         void* twp = tw ? tw->ptr : nullptr;
+        void* twrp = twr ? twr->ptr : nullptr;
         void* cp = chirp ? chirp->ptr : nullptr;
         void* bp = bh ? bh->ptr : nullptr;
         lines_desc dd = d;
         int inv = sign > 0 ? 1 : 0, nl = cfg.nlog;
-        void* args[] = {(void*)&in, &out, &twp, &cp, &bp, &dd, &inv, &nl};
+        void* args[] = {(void*)&in, &out, &twp, &twrp, &cp, &bp, &dd, &inv, &nl};
         return launch(k, grid, block, s, args);
     }
     if (cfg.kind != 0) {
@@ -566,7 +724,7 @@ bool parse_radices(const char* text, int n, std::vector<int>& out) {
         char* end = nullptr;
         const long r = std::strtol(p, &end, 10);
         if (end == p) return false;
-        if (r != 2 && r != 3 && r != 4 && r != 5 && r != 7 && r != 8 && r != 11 && r != 13 && r != 16) return false;
+        if (r < 2 || (r > 16 && !large_prime((int)r))) return false;
         out.push_back((int)r);
         prod *= r;
         p = end;
@@ -585,10 +743,11 @@ int32_t plan_fft_stage(int n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, i
                        int64_t out_ls, int64_t out_bs, int64_t out_ns, bool inplace, int effort,
                        hipStream_t stream, fft_stage* st, int lds_dma) {
     std::vector<int> rad;
-    if (!factorize(n, rad)) {
-        // a prime factor above 13, or more passes than a schedule holds: Bluestein
+    if (!factorize(n, rad) && !large_schedule(n, dbl, kMaxPrime(dbl), rad)) {
+        // a prime factor without a radix of its own, or more passes than a schedule holds:
+        // Bluestein
         fft_config c;
-        if (!any_config(0, n, dbl, false, c)) {
+        if (!any_config(0, n, dbl, false, (in_ns != 1 && in_ls == 1) || (out_ns != 1 && out_ls == 1), c)) {
             set_last_error("FFT length " + std::to_string(n) + ": the Bluestein work line does not fit in LDS");
             return DTFFT_HIP_ERROR_UNSUPPORTED_SIZE;
         }
@@ -596,7 +755,7 @@ int32_t plan_fft_stage(int n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, i
     }
     const bool in_cols = (in_ns != 1 && in_ls == 1);
     const bool out_cols = (out_ns != 1 && out_ls == 1);
-    fft_config cfg = default_fft_config(n, dbl, in_cols, out_cols, inplace);
+    fft_config cfg = default_fft_config(n, dbl, in_cols, out_cols, nl * nb, nl);
     lines_desc d = make_lines(nl, nb, in_ls, in_bs, in_ns, out_ls, out_bs, out_ns, cfg.lpb);
     char kb[256];
     std::snprintf(kb, sizeof kb, "fft|%d|%c|%d%d%d|%lld|%lld|%lld,%lld,%lld|%lld,%lld,%lld", n, dbl ? 'd' : 'f',
@@ -630,7 +789,7 @@ int32_t plan_fft_stage(int n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, i
         if (inplace) bo = bi;
         TRY(fill_tuning_scratch(bi, (size_t)si * es, dbl, stream));
         double best = 1e30;
-        auto cands = fft_candidates(n, dbl, in_cols, out_cols, inplace);
+        auto cands = fft_candidates(n, dbl, in_cols, out_cols, nl * nb, nl);
         if (effort < DTFFT_HIP_EXHAUSTIVE && cands.size() > 12) cands.resize(12);
         for (size_t i = 0, nc = cands.size(); lds_dma != 0 && i < nc; i++) {  // LDS-DMA twins
             for (int v : {1, 2}) {
@@ -684,8 +843,16 @@ int32_t plan_fft_stage(int n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, i
         // plain kernel, which the autotuner preferred there.
         fft_config c = cfg;
         c.dma = lds_dma == 2 ? 1 : lds_dma == 3 ? 2 : (c.out_cols ? 1 : 2);
+        c.staged = false;
         c.lpb = 128 / elem_bytes(dbl);  // a tile row is one 128-byte piece
-        if (c.out_cols && lds_dma < 2) c.tpl = std::max(1, c.tpl / 2);
+        // The radices as equal as they come, one butterfly per thread for powers of two from 256
+        // on, else 32 threads (320 = 8 8 5: 181 us per GiB, 198 us on 64; 192 = 16 12: 176, 184 us
+        // on 16).
+        if (factorize(n, c.radices)) {
+            const int t = n / *std::max_element(c.radices.begin(), c.radices.end());
+            c.tpl = n >= 256 && (n & (n - 1)) == 0 ? t : n <= 512 ? 32 : 64;
+        }
+        if (c.out_cols && lds_dma < 2 && n >= 256 && (n & (n - 1)) == 0) c.tpl = std::max(1, c.tpl / 2);
         bool wide = false;
         if (lds_dma == 1 && !dbl && inplace && cfg.out_cols && n >= 512) {
             // In-place FP32 column passes of n >= 512 where a 32-line tile (256-byte pieces of
@@ -724,26 +891,30 @@ int32_t plan_real_stage(int kind, int n, bool dbl, int64_t how_many, int64_t idi
     }
     const int m = n / 2;
     fft_config c;
-    if (n % 2 != 0 || !factorize(m, c.radices)) {
-        // odd lengths (directly when n factorizes) and halves with a prime factor above 13
-        // (Bluestein) take the any-length kernel: real side in real units
-        std::vector<int> rad;
+    // halves with a prime that is a radix of its own: only where the Bluestein form of n would fit
+    std::vector<int> rad;
+    const bool prime_ok = large_schedule(n, dbl, kMaxPrime(dbl), rad);
+    if (n % 2 != 0 || !(factorize(m, c.radices) || prime_ok)) {
+        // odd lengths (directly when n factorizes) and halves with a prime factor without a radix
+        // of its own (Bluestein) take the any-length kernel: real side in real units
         const bool direct = n % 2 != 0 && factorize(n, rad);
-        if (!any_config(kind, n, dbl, direct, c)) {
+        if (!any_config(kind, n, dbl, direct, false, c)) {
             set_last_error("R2C/C2R length " + std::to_string(n) + ": the work line does not fit in LDS");
             return DTFFT_HIP_ERROR_UNSUPPORTED_SIZE;
         }
         return st->init(c, make_lines(how_many, 1, idist, 0, 1, odist, 0, 1, c.lpb));
     }
-    c = default_fft_config(m, dbl, false, false, false);
+    c = default_fft_config(m, dbl, false, false, how_many, how_many);
+    c.staged = false;
     c.kind = kind;
     if (m == 1) {
         c.radices = {1}; c.tpl = 1; c.lpb = 64;
-    } else {
-        // one butterfly of the largest radix per thread and pass: the untangling adds
-        // registers to the row FFT, and fewer per thread keep more waves resident
-        const int rmax = *std::max_element(c.radices.begin(), c.radices.end());
-        if ((m / rmax) * c.lpb <= 1024) c.tpl = m / rmax;
+    } else if (factorize(m, rad)) {
+        // one butterfly per thread and pass: the untangling adds registers to the row FFT, and
+        // fewer per thread keep more waves resident
+        pick_schedule(m, 8, c.radices, c.tpl);
+        c.lpb = std::max(1, (c.tpl >= 64 ? 256 : 128) / c.tpl);
+        while (c.tpl > 1024) c.tpl = (c.tpl + 1) / 2;
     }
     lines_desc d;
     if (kind == 1) {  // real lines (idist reals) viewed as complex; complex out (odist)
@@ -765,17 +936,17 @@ int32_t plan_c2r_cols_stage(int n, bool dbl, int64_t nl, int64_t nb, int64_t in_
     }
     const int m = n / 2;
     fft_config c;
-    if (!factorize(m, c.radices) || m < 2) {
+    std::vector<int> rad;
+    if (!(factorize(m, c.radices) || large_schedule(n, dbl, kMaxPrime(dbl), rad)) || m < 2) {
         // Bluestein (or the direct form for n = 2) on the any-length kernel, which writes
         // real units: the strides of the complex view double
-        std::vector<int> rad;
-        if (!any_config(2, n, dbl, factorize(n, rad) && m < 2, c)) {
+        if (!any_config(2, n, dbl, factorize(n, rad) && m < 2, true, c)) {
             set_last_error("fused C2R length " + std::to_string(n) + ": the work line does not fit in LDS");
             return DTFFT_HIP_ERROR_UNSUPPORTED_SIZE;
         }
         return st->init(c, make_lines(nl, nb, 1, in_bs, in_ns, 2 * out_ls, 2 * out_bs, 1, c.lpb));
     }
-    c = default_fft_config(m, dbl, true, false, false);
+    c = default_fft_config(m, dbl, true, false, nl * nb, nl);
     c.kind = 2;
     lines_desc d = make_lines(nl, nb, 1, in_bs, in_ns, out_ls, out_bs, 1, c.lpb);
     // persistent blocks with both twiddle tables in LDS by the configuration's rule (FP32 by

@@ -105,6 +105,7 @@ struct fft_config {
     int dma = 0;  // column-in passes through LDS filled by direct loads: 1 double buffer
                   // (fft_cols_dma_kernel), 2 single buffer, two blocks per CU (fft_cols_dma1_kernel)
     int twl = 0;  // C2C (kind 0, dma 0): persistent blocks with the twiddle table in LDS
+    bool staged = false;  // C2C (kind 0, dma 0): the tile goes through LDS on its way in and out
     int oseg = 0;  // C2C and R2C rows (kind 0 / 1, dma 0): FFT axis written in chunks of `oseg` elements
     // fft_any_kernel (device/anylen.hip): any == 1 runs a line of logical length nlog through
     // the n-point schedule in LDS, directly (chirp false, n == nlog) or by Bluestein's chirp
@@ -126,17 +127,26 @@ int32_t get_twiddles(int n, const std::vector<int>& radices, bool dbl, std::shar
 int32_t get_bluestein(int n, int m, bool dbl, std::shared_ptr<twiddles>* chirp, std::shared_ptr<twiddles>* bh);
 // Configuration of fft_any_kernel for kind 0 / 1 / 2 of logical length n (Bluestein unless
 // `direct`, which needs n to factorize); false when the work line does not fit in LDS.
-bool any_config(int kind, int n, bool dbl, bool direct, fft_config& c);
+bool any_config(int kind, int n, bool dbl, bool direct, bool cols, fft_config& c);
 
+// The radix schedule of n (primes up to 13): fewest passes of radices up to 16.
 bool factorize(int n, std::vector<int>& radices);
+// The power-of-two part in the fewest radices of 16, 8, 4 and 2, then the odd primes up to 13.
+bool prime_schedule(int n, std::vector<int>& radices);
 // LDS bytes of the kernel a configuration names (tile, plus the LDS twiddle tables with twl).
 size_t fft_lds_bytes(const fft_config& c);
 // Sets c.twl by the rule of `mode` (0 never, 1 default rule, 2 wherever the kernel has the
 // form) for a stage of these lines, and only where the LDS budget allows it.
 void apply_twl(fft_config& c, const lines_desc& d, int mode);
-// Chooses tpl / lpb for a length and access mode (heuristic default of the autotuner).
-fft_config default_fft_config(int n, bool dbl, bool in_cols, bool out_cols, bool inplace);
-std::vector<fft_config> fft_candidates(int n, bool dbl, bool in_cols, bool out_cols, bool inplace);
+// Chooses schedule, tpl and lpb for a length and access mode (the default, and the autotuner's
+// first candidate); lines: how many the launch transforms (0: many), nl of them side by side.
+fft_config default_fft_config(int n, bool dbl, bool in_cols, bool out_cols, int64_t lines, int64_t nl);
+void pick_schedule(int n, int points, std::vector<int>& radices, int& tpl);
+std::vector<fft_config> fft_candidates(int n, bool dbl, bool in_cols, bool out_cols, int64_t lines, int64_t nl);
+// Schedules of lengths with prime factors above 13 that the kernels have as radices.
+bool large_schedule(int n, bool dbl, int max_prime, std::vector<int>& radices);
+// Largest such prime: in FP64 beyond 37 the registers of a butterfly no longer fit one wave.
+inline int kMaxPrime(bool dbl) { return dbl ? 37 : 61; }
 // Radix schedules of n for the autotuner (the default first), at most max_count.
 std::vector<std::vector<int>> radix_schedules(int n, int max_count);
 // Parses a tuning record's "r0,r1,..." schedule of n.
@@ -149,6 +159,7 @@ struct fft_stage {
     const rtc_kernel* k = nullptr;
     const rtc_kernel* k_alt = nullptr;  // cfg.dma: the plain column kernel, for misaligned buffers
     std::shared_ptr<twiddles> tw;
+    std::shared_ptr<twiddles> twr;  // cfg.chirp: the radices in reverse
     std::shared_ptr<twiddles> rtw;  // R2C / C2R untangling twiddles exp(-2 pi i k / 2M)
     std::shared_ptr<twiddles> chirp, bh;  // cfg.chirp: exp(-i pi j^2 / nlog), DFT_n(b) / n
     unsigned grid = 0, block = 0, grid_alt = 0;

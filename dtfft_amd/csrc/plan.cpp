@@ -135,8 +135,18 @@ static int32_t blocked_pair(plan_t* p, const fft_stage& rows, const fft_stage& c
                             fft_stage* cols_blk, bool* ok) {
     *ok = false;
     const fft_config& rc = rows.cfg;
-    const fft_config& cc = cols.cfg;
+    fft_config cc = cols.cfg;
     const int64_t es = (int64_t)p->cplx;
+    // chunks divide the lines; FP32 ones are whole 128-byte pieces, also where so few lines run
+    // that the natural pass takes tiles of 8
+    if (!cc.dma) {
+        while (cc.lpb > 8 && cols.d.nl % cc.lpb != 0) cc.lpb /= 2;
+        if (!p->dbl && cc.lpb < 16 && cc.tpl * 16 <= 1024) {
+            cc.lpb = 16;
+            if (fft_lds_bytes(cc) > 64 * 1024) cc.lpb = 8;
+        }
+    }
+    if (!p->dbl && cc.lpb % 16 != 0) return DTFFT_HIP_SUCCESS;
     if (!global_config().blocked || !rows.k || !cols.k) return DTFFT_HIP_SUCCESS;
     if (rc.kind != 0 || rc.any || rc.dma || rc.seg || rc.in_cols || rc.out_cols || rc.n <= 1) return DTFFT_HIP_SUCCESS;
     if (cc.kind != 0 || cc.any || !cc.in_cols || cc.out_cols || cc.seg || cc.n <= 1) return DTFFT_HIP_SUCCESS;
@@ -171,7 +181,7 @@ static int32_t blocked_pair(plan_t* p, const fft_stage& rows, const fft_stage& c
 
 // Chunk-blocked pair of the fused 3D R2C forward: the R2C rows write the complex X-pencil in
 // chunks of B lines (element (x, y) of plane z at z * ncp * ny + (x / B) * ny * B + y * B +
-// x % B), padded to ncp = ceil(nc / B) * B lines, so that the X->Y pass reads whole contiguous
+// x % B), padded to ncp = ceil(nc / 16) * 16 lines, so that the X->Y pass reads whole contiguous
 // tiles (FP32: by LDS DMA) although nc = nx / 2 + 1 lines do not divide into them (nor do rows
 // of nc complex values align to 16 bytes).  The padding lines of the last chunk are never
 // written; the X->Y pass transforms them into planes x >= nc of the Y-pencil in aux, which the
@@ -179,18 +189,19 @@ static int32_t blocked_pair(plan_t* p, const fft_stage& rows, const fft_stage& c
 // plan's buffers grow to ncp * ny * nz complex values).
 static int32_t blocked_r2c(plan_t* p, bool* ok) {
     *ok = false;
-    const int64_t ny = p->ny, nz = p->nz, nc = p->nc, B = 16;
+    const int64_t ny = p->ny, nz = p->nz, nc = p->nc;
     const fft_config& rc = p->fx.cfg;
     if (!global_config().blocked || !p->fx.k || rc.kind != 1 || rc.any || rc.dma)
         return DTFFT_HIP_SUCCESS;  // the half-length R2C row kernel (fft_r2c_kernel) only
-    const int64_t ncp = (nc + B - 1) / B * B;
+    const int64_t ncp = (nc + 15) / 16 * 16;
     if ((ncp - nc) * 16 > nc) return DTFFT_HIP_SUCCESS;
     fft_stage nat;  // the X->Y pass over the padded rows in the natural layout: its configuration
     TRY(fused(p, ny, ncp, nz, ncp * ny, ncp, ny * nz, ny, &nat));
-    // the column pass's tile is B lines: FP32 the LDS-DMA kernel (128-byte pieces), FP64 the
-    // plain column kernel (256-byte pieces)
+    // the column pass's tile is B lines (a divisor of 16): FP32 the LDS-DMA kernel, FP64 the plain
+    // column kernel
     const fft_config& cc = nat.cfg;
-    if (!nat.k || cc.kind != 0 || cc.any || !cc.in_cols || cc.out_cols || cc.seg || cc.lpb != B)
+    const int64_t B = cc.lpb;
+    if (!nat.k || cc.kind != 0 || cc.any || !cc.in_cols || cc.out_cols || cc.seg || 16 % B != 0)
         return DTFFT_HIP_SUCCESS;
     lines_desc bd = nat.d;
     bd.in_ns = B;

@@ -31,7 +31,7 @@ int r2r_inverse_kind(int kind) {  // src/dtfft_utils.F90:447-471
 // M = 256 against 117).
 static bool half_schedule(int m, std::vector<int>& out) {
     std::vector<int> f;
-    if (!factorize(m, f)) return false;
+    if (!prime_schedule(m, f)) return false;
     int p2 = 0, rest = m;
     while (rest % 2 == 0) { rest /= 2; p2++; }
     out.assign((size_t)(p2 / 2), 4);
@@ -82,7 +82,7 @@ int32_t r2r_stage::init(int kind_, int64_t n_, bool dbl_, int64_t nl, int64_t nb
                          half_schedule((int)(n / 2), hrad);
     const int64_t mf = half_ok ? n / 2 : m;  // length of the fused kernel's FFT
     if ((factors || half_ok) && in_es == 1 && out_es == 1 && in_ls == out_ls && in_bs == out_bs && even && m > 1) {
-        fft_config c = default_fft_config((int)mf, dbl, false, false, false);
+        fft_config c = default_fft_config((int)mf, dbl, false, false, nl * nb, nl);
         if (half_ok) {
             // M / 4 threads per line (one butterfly of radix <= 4 per pass), 512-thread blocks.
             // Measured on MI355X at 512^3 FP32 (medians of interleaved rounds), DCT-2 / DCT-3
@@ -94,9 +94,10 @@ int32_t r2r_stage::init(int kind_, int64_t n_, bool dbl_, int64_t nl, int64_t nb
             c.tpl = (int)std::max<int64_t>(1, mf / std::max(4, rmax));
             c.lpb = std::max(1, 512 / c.tpl);
         } else {
-            // one butterfly of the largest radix per thread and pass
-            const int rmax = *std::max_element(c.radices.begin(), c.radices.end());
-            if ((mf / rmax) * c.lpb <= 1024) c.tpl = (int)(mf / rmax);
+            // one butterfly per thread and pass, two waves per block
+            pick_schedule((int)mf, 8, c.radices, c.tpl);
+            c.lpb = std::max(1, 128 / c.tpl);
+            while (c.tpl * c.lpb > 1024) c.tpl = (c.tpl + 1) / 2;
         }
         const size_t ec = dbl ? 16 : 8, er = dbl ? 8 : 4;
         // work lines, real lines, FFT twiddles (mf - 1 of 16 bytes), table (2n complex), and
@@ -192,7 +193,7 @@ int32_t r2r_stage::init_cols(int kind_, int64_t n_, bool dbl_, int64_t nl, int64
     const int lpb = (int)(128 / er);  // a tile row is one 128-byte piece of LPB reals
     if (nl % lpb != 0) return DTFFT_HIP_SUCCESS;
     const int64_t mf = n_ / 2;
-    fft_config c = default_fft_config((int)mf, dbl_, false, false, false);
+    fft_config c = default_fft_config((int)mf, dbl_, false, false, 0, 0);
     c.radices = hrad;
     c.pad = 1;
     c.lpb = lpb;
