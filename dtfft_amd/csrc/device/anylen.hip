@@ -31,102 +31,6 @@
 // exchanges, M = R0 R1 R2 four.
 #include "fft.hip"
 
-namespace dtfft {
-// Passes of S with N / R butterflies spread over TPL threads of a line, elements taken from and
-// given to functors: load(line, n) and store(line, n, value).
-template <typename T, class S, int TPL, int LPB>
-struct any_passes {
-    typedef typename tw_of<T>::type tw_t;
-    static constexpr int NT = TPL * LPB;
-
-    template <bool COLS>
-    static __device__ __forceinline__ void map(int& line, int& j) {
-        if (COLS) { line = threadIdx.x % LPB; j = threadIdx.x / LPB; }
-        else { line = threadIdx.x / TPL; j = threadIdx.x % TPL; }
-    }
-
-    // pass p; BAR: a barrier between the last load and the first store (in place in LDS)
-    template <int p, bool COLS, bool BAR, class Load, class Store>
-    static __device__ __forceinline__ void run(const tw_t* __restrict__ tw, const Load& load, const Store& store) {
-        constexpr int R = S::radix(p), L = S::span(p), TWO = S::tw_off(p);
-        constexpr int NB = S::N / R, IT = (NB + TPL - 1) / TPL;
-        int line, j;
-        map<COLS>(line, j);
-        cx<T> v[IT][R];
-#pragma unroll
-        for (int it = 0; it < IT; it++) {
-            const int b = j + it * TPL;
-            if (IT * TPL == NB || b < NB) {
-#pragma unroll
-                for (int r = 0; r < R; r++) v[it][r] = load(line, b + r * NB);
-            }
-        }
-        if (BAR) __syncthreads();
-#pragma unroll
-        for (int it = 0; it < IT; it++) {
-            const int b = j + it * TPL;
-            if (IT * TPL == NB || b < NB) {
-                const int k = b % L;
-                if (L > 1) {
-#pragma unroll
-                    for (int r = 1; r < R; r++) v[it][r] = twmul(v[it][r], tw[TWO + k * (R - 1) + (r - 1)]);
-                }
-                bfly<T, R>::run(v[it]);
-#pragma unroll
-                for (int s = 0; s < R; s++) store(line, (b - k) * R + k + s * L, v[it][s]);
-            }
-        }
-    }
-
-    // The last pass of S, the product with bh and the conjugation, and the first pass of the
-    // reversed schedule, in place in LDS (line stride LD).
-    template <int LD>
-    static __device__ __forceinline__ void turn(const tw_t* __restrict__ tw, const tw_t* __restrict__ bh, cx<T>* lds) {
-        constexpr int p = S::NP - 1;
-        constexpr int R = S::radix(p), TWO = S::tw_off(p);
-        constexpr int NB = S::N / R, IT = (NB + TPL - 1) / TPL;
-        static_assert(S::span(p) == NB, "the last pass");
-        int line, j;
-        map<false>(line, j);
-        cx<T> v[IT][R];
-#pragma unroll
-        for (int it = 0; it < IT; it++) {
-            const int b = j + it * TPL;
-            if (IT * TPL == NB || b < NB) {
-#pragma unroll
-                for (int r = 0; r < R; r++) v[it][r] = lds[line * LD + b + r * NB];
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int it = 0; it < IT; it++) {
-            const int b = j + it * TPL;
-            if (IT * TPL == NB || b < NB) {
-#pragma unroll
-                for (int r = 1; r < R; r++) v[it][r] = twmul(v[it][r], tw[TWO + b * (R - 1) + (r - 1)]);
-                bfly<T, R>::run(v[it]);
-#pragma unroll
-                for (int s = 0; s < R; s++) v[it][s] = conj(twmul(v[it][s], bh[b + s * NB]));
-                bfly<T, R>::run(v[it]);
-#pragma unroll
-                for (int s = 0; s < R; s++) lds[line * LD + b * R + s] = v[it][s];
-            }
-        }
-    }
-
-    // passes p .. p_end - 1 in place in LDS, a barrier after each
-    template <int p, int p_end, int LD>
-    static __device__ __forceinline__ void inner(const tw_t* __restrict__ tw, cx<T>* lds) {
-        if constexpr (p < p_end) {
-            auto ld = [&](int line, int n) { return lds[line * LD + n]; };
-            auto st = [&](int line, int n, cx<T> y) { lds[line * LD + n] = y; };
-            run<p, false, true>(tw, ld, st);
-            __syncthreads();
-            inner<p + 1, p_end, LD>(tw, lds);
-        }
-    }
-};
-}  // namespace dtfft
 
 // S: the schedule of M; SR: its radices in reverse (CHIRP only, with the table twr).
 // IN_COLS / OUT_COLS: lines adjacent in memory on that side, so threads run across lines.
@@ -137,8 +41,8 @@ fft_any_kernel(const void* __restrict__ in_, void* __restrict__ out_,
                const typename tw_of<T>::type* __restrict__ twr_,
                const typename tw_of<T>::type* __restrict__ chirp_,
                const typename tw_of<T>::type* __restrict__ bh_, dtfft::lines_desc d, int inv, int n) {
-    typedef dtfft::any_passes<T, S, TPL, LPB> F;
-    typedef dtfft::any_passes<T, SR, TPL, LPB> B;
+    typedef dtfft::line_passes<T, S, TPL, LPB> F;
+    typedef dtfft::line_passes<T, SR, TPL, LPB> B;
     constexpr int NP = S::NP, LD = S::N + PAD;
     __shared__ cx<T> lds[LPB * LD];
     const bool iv = KIND == 2 ? true : (KIND == 1 ? false : inv != 0);

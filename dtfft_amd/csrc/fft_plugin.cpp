@@ -285,6 +285,13 @@ void pick_schedule(int n, int points, std::vector<int>& radices, int& tpl) {
     if (radices.size() == 2) { tpl = n / radices[1]; return; }
     tpl = 16;
     while (n > tpl * points) tpl *= 2;
+    static std::mutex mu;
+    static std::map<std::pair<int, int>, std::vector<int>> known;  // (n, tpl)
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        auto it = known.find({n, tpl});
+        if (it != known.end()) { radices = it->second; return; }
+    }
     const size_t np = radices.size();
     std::vector<int> cur;
     double best = 1e30;
@@ -304,6 +311,8 @@ void pick_schedule(int n, int points, std::vector<int>& radices, int& tpl) {
             }
     };
     rec(n, 16);
+    std::lock_guard<std::mutex> lk(mu);
+    known[{n, tpl}] = radices;
 }
 
 fft_config default_fft_config(int n, bool dbl, bool in_cols, bool out_cols, int64_t lines, int64_t nl) {

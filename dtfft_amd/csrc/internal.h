@@ -206,7 +206,8 @@ struct r2r_stage {
     std::shared_ptr<twiddles> ftw;  // twiddles of the length-m FFT
     std::shared_ptr<twiddles> t4;   // e^{-i pi j / 4n}, j < 2n
     std::shared_ptr<twiddles> rtw;  // half-length form: e^{-2 pi i k / n}, k <= n / 2
-    bool half = false;              // fused kernel runs types 2 / 3 through an n/2-point FFT
+    bool half = false;              // half-length form (device/r2r.hip)
+    bool tile = false;              // fused through r2r_tile_kernel: any strides, partial tiles
     unsigned fgrid = 0, fblock = 0;
     int32_t init(int kind, int64_t n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, int64_t in_bs,
                  int64_t in_es, int64_t out_ls, int64_t out_bs, int64_t out_es, int effort, hipStream_t stream);
@@ -217,6 +218,11 @@ struct r2r_stage {
     // multiple of the 128-byte tile row.
     int32_t init_cols(int kind, int64_t n, bool dbl, int64_t nl, int64_t nb, int64_t in_bs, int64_t in_es,
                       int64_t out_ls, int64_t out_bs, int64_t out_es, bool out_cols, bool* ok);
+    // One launch of r2r_tile_kernel for any strides on both sides (in place where they are equal);
+    // *ok is false (nothing set up) where the work length has a prime without a radix or the
+    // tile does not fit.
+    int32_t init_tile(int kind, int64_t n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, int64_t in_bs,
+                      int64_t in_es, int64_t out_ls, int64_t out_bs, int64_t out_es, bool* ok);
     // Chunk-blocked pair (fused kernels, half-length form): `rows` writing its lines (nl
     // lines of nb batches, rows of n) in chunks of B elements -- element k of line (l, b) at
     // b * n * nl + l * B + (k / B) * nl * B + k % B -- so that the column stage `cols` (B lines

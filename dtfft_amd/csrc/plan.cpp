@@ -77,6 +77,10 @@ struct plan_t {
     // (3D) / ryb -> rxbc (2D)
     r2r_stage rx_blk, ryc_blk, rb_blk, rbc_blk;
     bool r2r_blk_fwd = false, r2r_blk_bwd = false;
+    // otherwise: column stages of r2r_tile_kernel, axis by axis where they exist (the axes
+    // without one take a permute and the row stage)
+    r2r_stage cy, cz, cxb, cyb;
+    bool r2r_cols = false, has_cy = false, has_cz = false, has_cxb = false, has_cyb = false;
     void* work = nullptr;                            // complex work lines of the R2R stages
     // forward + backward captured as one hipGraph for one set of pointers
     hipStream_t gstream = nullptr;
@@ -272,6 +276,23 @@ static int32_t build_r2r(plan_t* p) {
                 TRY(r2r_stage::blocked_pair(p->rx, p->ryc, &p->rx_blk, &p->ryc_blk, &p->r2r_blk_fwd));
                 TRY(r2r_stage::blocked_pair(p->ryb, p->rxbc, &p->rb_blk, &p->rbc_blk, &p->r2r_blk_bwd));
             }
+        }
+        if (!p->r2r_fused) {
+            // The same order with the general column stages: forward X rows, X->Y + Y, Y->Z + Z;
+            // backward Z rows, Z->X + X, Y in place on the X-pencil.
+            if (p->ndims == 3) {
+                const int k2 = p->kind[2];
+                TRY(p->cy.init_tile(k1, ny, p->dbl, nx, nz, 1, nx * ny, nx, ny * nz, ny, 1, &p->has_cy));
+                TRY(p->cz.init_tile(k2, nz, p->dbl, ny, nx, 1, ny * nz, ny, nz * nx, nz, 1, &p->has_cz));
+                TRY(p->cxb.init_tile(i0, nx, p->dbl, nz, ny, 1, nz * nx, nz, nx * ny, nx, 1, &p->has_cxb));
+                TRY(p->cyb.init_tile(i1, ny, p->dbl, nx, nz, 1, nx * ny, nx, 1, nx * ny, nx, &p->has_cyb));
+                if (!p->has_cxb)  // Z (nz, nx, ny) -> X (nx, ny, nz)
+                    TRY(p->t_zx.create(DTFFT_HIP_KERNEL_PERMUTE_FORWARD, 3, nz, nx, ny, (int)p->cplx, E));
+            } else {
+                TRY(p->cy.init_tile(k1, ny, p->dbl, nx, 1, 1, 0, nx, ny, 0, 1, &p->has_cy));
+                TRY(p->cxb.init_tile(i0, nx, p->dbl, ny, 1, 1, 0, ny, nx, 0, 1, &p->has_cxb));
+            }
+            p->r2r_cols = p->has_cy || p->has_cz || p->has_cxb;
         }
     }
     return DTFFT_HIP_SUCCESS;
@@ -509,6 +530,53 @@ static int32_t exec_r2r(plan_t* p, void* in, void* out, bool fwd, void* aux, ste
             STEP(r, (bb ? p->rbc_blk : p->rxbc).run(aux, out, w, s));
             STEP(r, p->rybc.run(out, out, w, s));
         }
+        return DTFFT_HIP_SUCCESS;
+    }
+    if (p->r2r_cols && p->ndims == 2) {
+        if (fwd) {
+            STEP(r, p->rx.run(in, aux, w, s));
+            if (p->has_cy) {
+                STEP(r, p->cy.run(aux, out, w, s));
+            } else {
+                STEP(r, p->t_xy.run(aux, out, s));
+                STEP(r, p->ry.run(out, out, w, s));
+            }
+        } else {
+            STEP(r, p->ryb.run(in, aux, w, s));
+            if (p->has_cxb) {
+                STEP(r, p->cxb.run(aux, out, w, s));
+            } else {
+                STEP(r, p->t_yx.run(aux, out, s));
+                STEP(r, p->rxb.run(out, out, w, s));
+            }
+        }
+        return DTFFT_HIP_SUCCESS;
+    }
+    if (p->r2r_cols && fwd) {
+        STEP(r, p->rx.run(in, out, w, s));
+        if (p->has_cy) {
+            STEP(r, p->cy.run(out, aux, w, s));
+        } else {
+            STEP(r, p->t_xy.run(out, aux, s));
+            STEP(r, p->ry.run(aux, aux, w, s));
+        }
+        if (p->has_cz) {
+            STEP(r, p->cz.run(aux, out, w, s));
+        } else {
+            STEP(r, p->t_yz.run(aux, out, s));
+            STEP(r, p->rz.run(out, out, w, s));
+        }
+        return DTFFT_HIP_SUCCESS;
+    }
+    if (p->r2r_cols && p->has_cyb) {
+        STEP(r, p->rzb.run(in, aux, w, s));
+        if (p->has_cxb) {
+            STEP(r, p->cxb.run(aux, out, w, s));
+        } else {
+            STEP(r, p->t_zx.run(aux, out, s));
+            STEP(r, p->rxb.run(out, out, w, s));
+        }
+        STEP(r, p->cyb.run(out, out, w, s));
         return DTFFT_HIP_SUCCESS;
     }
     if (p->ndims == 2) {
@@ -829,6 +897,10 @@ int32_t dtfft_hip_report(dtfft_hip_plan_t plan) {
         show_r2r("r2r_ycol", p->rybc);
         if (p->r2r_blk_fwd) { show_r2r("r2r_frow", p->rx_blk); show_r2r("r2r_fcol", p->ryc_blk); }
         if (p->r2r_blk_bwd) { show_r2r("r2r_brow", p->rb_blk); show_r2r("r2r_bcol", p->rbc_blk); }
+    }
+    if (p->r2r_cols) {
+        show_r2r("r2r_y", p->cy); show_r2r("r2r_z", p->cz); show_r2r("r2r_xb", p->cxb);
+        show_r2r("r2r_ycb", p->cyb);
     }
     auto show = [](const char* name, const fft_stage& st) {
         if (!st.k) return;

@@ -3,8 +3,9 @@
 // 149-223) or VkFFT (src/interfaces/fft/vkfft/dtfft_executor_vkfft_m.F90:97-123).  A stage
 // is r2r_pre (real line -> complex line of length M), the Stockham C2C transform of the
 // work line, and r2r_post (complex -> n real outputs); device/r2r.hip lists the per-kind
-// maps.  Contiguous lines run all three in one kernel through LDS; other layouts run three
-// launches through a work buffer (lines x M complex) that belongs to the caller.
+// maps.  One kernel runs all three through LDS (init, init_cols: persistent, types 2 and 3 of even
+// length; init_tile: every kind and layout); work lengths without a schedule run three launches
+// through a work buffer (lines x M complex) that belongs to the caller.
 #include <map>
 #include <mutex>
 
@@ -41,11 +42,28 @@ static bool half_schedule(int m, std::vector<int>& out) {
     return out.size() <= 10;
 }
 
+// Half-length forms (device/r2r.hip): types 1 of three points and more (DST-1 of any), the others
+// of even length.
+static bool half_form(int kind, int64_t n) {
+    if (kind == 3) return n >= 3;
+    if (kind == 7) return n >= 1;
+    return n >= 4 && n % 2 == 0;
+}
+
 static int64_t work_length(int kind, int64_t n) {
-    if (kind == 3) return 2 * (n - 1);
-    if (kind == 7) return 2 * (n + 1);
-    if (kind == 6 || kind == 10) return 2 * n;
-    return n;
+    if (kind == 3) return half_form(kind, n) ? n - 1 : 2 * (n - 1);
+    if (kind == 7) return n + 1;
+    if (half_form(kind, n)) return n / 2;
+    return kind == 6 || kind == 10 ? 2 * n : n;
+}
+
+// Lengths that the stages take: the full-length work line (2(n-1), 2(n+1), 2n or n points) fits the
+// LDS of a block, by itself or, with a prime above 13, as Bluestein's line.
+static bool length_taken(int kind, int64_t n, bool dbl) {
+    const int64_t full = kind == 3 ? 2 * (n - 1) : kind == 7 ? 2 * (n + 1) : (kind == 6 || kind == 10) ? 2 * n : n;
+    const int64_t most = 160 * 1024 / (dbl ? 16 : 8);
+    std::vector<int> r;
+    return full <= most && (prime_schedule((int)full, r) || 2 * full - 1 <= most);
 }
 
 int32_t r2r_stage::init(int kind_, int64_t n_, bool dbl_, int64_t nl, int64_t nb, int64_t in_ls, int64_t in_bs,
@@ -59,66 +77,64 @@ int32_t r2r_stage::init(int kind_, int64_t n_, bool dbl_, int64_t nl, int64_t nb
         set_last_error("R2R length " + std::to_string(n_) + " too short for kind " + std::to_string(kind_));
         return DTFFT_HIP_ERROR_UNSUPPORTED_SIZE;
     }
+    if (!length_taken(kind_, n_, dbl_)) {
+        set_last_error("R2R length " + std::to_string(n_) + ": the work line does not fit in LDS");
+        return DTFFT_HIP_ERROR_UNSUPPORTED_SIZE;
+    }
     kind = kind_;
     n = n_;
     dbl = dbl_;
     m = work_length(kind, n);
+    half = half_form(kind, n);
     d = r2r_desc_h{nl, nb, in_ls, in_bs, in_es, out_ls, out_bs, out_es, n, m, m};
     const std::string t = dbl ? "double" : "float";
     // types 3 (DCT-3, DST-3) run the backward transform
     sign = (kind == 4 || kind == 8) ? DTFFT_HIP_FFT_BACKWARD : DTFFT_HIP_FFT_FORWARD;
-    // A work length with a prime factor above 13 runs the three launches, whose C2C stage
-    // is then the Bluestein form of plan_fft_stage.
-    std::vector<int> rad;
-    const bool factors = factorize((int)m, rad);
-    // One kernel for unit-stride, evenly spaced lines whose output overwrites nothing but the
-    // line itself: a block reads its lines whole before writing them, so in place is safe.
-    // Batches that continue the line spacing fold into one range of lines.
+    // Types 2 and 3 of even length over unit-stride, evenly spaced lines: the persistent kernel.
+    // A block reads its lines whole before writing them, so in place is safe.  Batches that
+    // continue the line spacing fold into one range of lines.
     const bool even = nb == 1 || (in_bs == nl * in_ls && out_bs == nl * out_ls);
-    // Types 2 and 3 of even length run the fused kernel's half-length form: the n-point
-    // transform of a real sequence (or of a Hermitian spectrum) as an n/2-point one.
     std::vector<int> hrad;
     const bool half_ok = (kind == 4 || kind == 5 || kind == 8 || kind == 9) && n % 2 == 0 && n >= 8 &&
                          half_schedule((int)(n / 2), hrad);
-    const int64_t mf = half_ok ? n / 2 : m;  // length of the fused kernel's FFT
-    if ((factors || half_ok) && in_es == 1 && out_es == 1 && in_ls == out_ls && in_bs == out_bs && even && m > 1) {
+    const int64_t mf = n / 2;  // length of its FFT
+    bool ok = false;
+    if ((n & (n - 1)) != 0) {
+        // the persistent kernel below, with its radix-4 passes, is the faster form for powers of
+        // two only (512 MB FP32 DCT-2 / DCT-3 rows: 128 points 253 / 209 us against 280 / 228;
+        // 384 points 422 / 395 us against 333 / 285)
+        TRY(init_tile(kind, n, dbl, nl, nb, in_ls, in_bs, in_es, out_ls, out_bs, out_es, &ok));
+        if (ok) return DTFFT_HIP_SUCCESS;
+    }
+    if (half_ok && in_es == 1 && out_es == 1 && in_ls == out_ls && in_bs == out_bs && even) {
         fft_config c = default_fft_config((int)mf, dbl, false, false, nl * nb, nl);
-        if (half_ok) {
-            // M / 4 threads per line (one butterfly of radix <= 4 per pass), 512-thread blocks.
-            // Measured on MI355X at 512^3 FP32 (medians of interleaved rounds), DCT-2 / DCT-3
-            // stage: 269 / 239 us with 8 lines of 64 threads, 297 / 254 us with 4 lines,
-            // 306 / 232 us with radix-8 passes at 32 threads per line, 328 / 314 us for the
-            // full-length form.
-            c.radices = hrad;
-            const int rmax = *std::max_element(hrad.begin(), hrad.end());
-            c.tpl = (int)std::max<int64_t>(1, mf / std::max(4, rmax));
-            c.lpb = std::max(1, 512 / c.tpl);
-        } else {
-            // one butterfly per thread and pass, two waves per block
-            pick_schedule((int)mf, 8, c.radices, c.tpl);
-            c.lpb = std::max(1, 128 / c.tpl);
-            while (c.tpl * c.lpb > 1024) c.tpl = (c.tpl + 1) / 2;
-        }
+        // M / 4 threads per line (one butterfly of radix <= 4 per pass), 512-thread blocks.
+        // Measured on MI355X at 512^3 FP32 (medians of interleaved rounds), DCT-2 / DCT-3
+        // stage: 269 / 239 us with 8 lines of 64 threads, 297 / 254 us with 4 lines,
+        // 306 / 232 us with radix-8 passes at 32 threads per line, 328 / 314 us for the
+        // full-length form.
+        c.radices = hrad;
+        const int rmax = *std::max_element(hrad.begin(), hrad.end());
+        c.tpl = (int)std::max<int64_t>(1, mf / std::max(4, rmax));
+        c.lpb = std::max(1, 512 / c.tpl);
         const size_t ec = dbl ? 16 : 8, er = dbl ? 8 : 4;
         // work lines, real lines, FFT twiddles (mf - 1 of 16 bytes), table (2n complex), and
-        // the half-length form's untangling table (n/2 + 1 of 16 bytes)
+        // the untangling table (n/2 + 1 of 16 bytes)
         const size_t lds = (size_t)c.lpb * (size_t)(c.n + c.pad) * ec + (size_t)c.lpb * n * er +
                            (size_t)std::max<int64_t>(1, mf - 1) * 16 + (size_t)(2 * n) * ec +
-                           (half_ok ? (size_t)(n / 2 + 1) * 16 : 16);
+                           (size_t)(n / 2 + 1) * 16;
         if (lds <= 160 * 1024) {
             d = r2r_desc_h{nl * nb, 1, in_ls, nl * nb * in_ls, 1, out_ls, nl * nb * out_ls, 1, n, m, m};
             std::string e = "fft_r2r_kernel<" + t + ", dtfft::sched<" + std::to_string(mf);
             for (int r : c.radices) e += ", " + std::to_string(r);
             e += ">, " + std::to_string(c.tpl) + ", " + std::to_string(c.lpb) + ", " + std::to_string(c.pad) + ", " +
-                 std::to_string(kind) + ((nl * nb) % c.lpb == 0 ? ", true" : ", false") +
-                 (half_ok ? ", true>" : ">");
+                 std::to_string(kind) + ((nl * nb) % c.lpb == 0 ? ", true>" : ", false>");
             TRY(rtc_get("r2r", e, &fk));
             expr = e;
             lpb = c.lpb;
             TRY(get_twiddles((int)mf, c.radices, dbl, &ftw));
             TRY(get_r2r_table(n, dbl, &t4));
-            if (half_ok) TRY(get_rtwiddles((int)n, dbl, &rtw));
-            half = half_ok;
+            TRY(get_rtwiddles((int)n, dbl, &rtw));
             const int64_t tiles = (nl * nb + c.lpb - 1) / c.lpb;
             fblock = (unsigned)(c.tpl * c.lpb);
             // persistent: as many blocks as are resident
@@ -133,9 +149,72 @@ int32_t r2r_stage::init(int kind_, int64_t n_, bool dbl_, int64_t nl, int64_t nb
             return DTFFT_HIP_SUCCESS;
         }
     }
-    TRY(rtc_get("r2r", "r2r_pre<" + t + ", " + std::to_string(kind) + ">", &pre));
-    TRY(rtc_get("r2r", "r2r_post<" + t + ", " + std::to_string(kind) + ">", &post));
+    TRY(init_tile(kind, n, dbl, nl, nb, in_ls, in_bs, in_es, out_ls, out_bs, out_es, &ok));
+    if (ok) return DTFFT_HIP_SUCCESS;
+    // A work length with a prime that no radix covers (or one that does not fit) runs three
+    // launches, whose C2C stage is the Bluestein form of plan_fft_stage.
+    const std::string h = half ? ", true>" : ", false>";
+    TRY(rtc_get("r2r", "r2r_pre<" + t + ", " + std::to_string(kind) + h, &pre));
+    TRY(rtc_get("r2r", "r2r_post<" + t + ", " + std::to_string(kind) + h, &post));
     return plan_fft_stage((int)m, dbl, nl * nb, 1, m, 0, 1, m, 0, 1, true, effort, stream, &fft);
+}
+
+int32_t r2r_stage::init_tile(int kind_, int64_t n_, bool dbl_, int64_t nl, int64_t nb, int64_t in_ls, int64_t in_bs,
+                             int64_t in_es, int64_t out_ls, int64_t out_bs, int64_t out_es, bool* ok) {
+    *ok = false;
+    if (!r2r_kind_valid(kind_) || n_ < 1 || (kind_ == 3 && n_ < 2) || !length_taken(kind_, n_, dbl_))
+        return DTFFT_HIP_SUCCESS;
+    const int64_t M = work_length(kind_, n_);
+    fft_config c;
+    if (M < 2) return DTFFT_HIP_SUCCESS;
+    c.n = (int)M;
+    c.dbl = dbl_;
+    c.pad = 1;
+    if (large_schedule((int)M, dbl_, kMaxPrime(dbl_), c.radices))
+        c.tpl = (int)std::max(M / c.radices[0], (M + 23) / 24);
+    else if (factorize((int)M, c.radices))
+        pick_schedule((int)M, 8, c.radices, c.tpl);
+    else
+        return DTFFT_HIP_SUCCESS;
+    // rows (on both sides): batches that continue the line spacing are one range of lines
+    const bool ic = in_ls == 1 && in_es != 1, oc = out_ls == 1 && out_es != 1;
+    if (!ic && !oc && in_bs == nl * in_ls && out_bs == nl * out_ls) { nl *= nb; nb = 1; }
+    if (ic || oc) {
+        // 128-byte pieces of reals where the tile leaves room for four blocks per CU, and no
+        // wider than the lines or than two tiles per CU need
+        c.lpb = dbl_ ? 16 : 32;
+        while (c.lpb > 8 && (fft_lds_bytes(c) > 40 * 1024 || c.tpl * c.lpb > 1024 || c.lpb >= 2 * nl ||
+                             (c.tpl * c.lpb >= 128 && nl * nb / c.lpb < 512)))
+            c.lpb /= 2;
+    } else {
+        c.lpb = std::max(1, (c.tpl >= 128 ? 256 : 128) / c.tpl);
+        while (c.lpb > 1 && c.tpl * c.lpb >= 128 && nl * nb / c.lpb < 512) c.lpb /= 2;
+    }
+    while (c.lpb > 1 && (fft_lds_bytes(c) > 160 * 1024 || c.tpl * c.lpb > 1024)) c.lpb /= 2;
+    while (c.tpl > 1024) c.tpl = (c.tpl + 1) / 2;
+    if (fft_lds_bytes(c) > 160 * 1024) return DTFFT_HIP_SUCCESS;
+    kind = kind_;
+    n = n_;
+    dbl = dbl_;
+    m = M;
+    half = half_form(kind, n);
+    sign = (kind == 4 || kind == 8) ? DTFFT_HIP_FFT_BACKWARD : DTFFT_HIP_FFT_FORWARD;
+    d = r2r_desc_h{nl, nb, in_ls, in_bs, in_es, out_ls, out_bs, out_es, n, m, m};
+    std::string e = std::string("r2r_tile_kernel<") + (dbl ? "double" : "float") + ", dtfft::sched<" + std::to_string(m);
+    for (int r : c.radices) e += ", " + std::to_string(r);
+    e += ">, " + std::to_string(c.tpl) + ", " + std::to_string(c.lpb) + ", " + std::to_string(c.pad) + ", " +
+         std::to_string(kind) + (half ? ", true" : ", false") + (ic ? ", true" : ", false") + (oc ? ", true>" : ", false>");
+    TRY(rtc_get("r2r", e, &fk));
+    expr = e;
+    lpb = c.lpb;
+    TRY(get_twiddles((int)m, c.radices, dbl, &ftw));
+    TRY(get_r2r_table(n, dbl, &t4));
+    TRY(get_rtwiddles((int)(2 * m), dbl, &rtw));
+    fblock = (unsigned)(c.tpl * c.lpb);
+    fgrid = (unsigned)std::min<int64_t>((nl + c.lpb - 1) / c.lpb * nb, 1 << 22);
+    fused = tile = true;
+    *ok = true;
+    return DTFFT_HIP_SUCCESS;
 }
 
 int32_t r2r_stage::blocked_pair(const r2r_stage& rows, const r2r_stage& cols, r2r_stage* rows_blk,
@@ -143,14 +222,14 @@ int32_t r2r_stage::blocked_pair(const r2r_stage& rows, const r2r_stage& cols, r2
     *ok = false;
     if (!global_config().blocked) return DTFFT_HIP_SUCCESS;
     // rows: the fused half-length row form over evenly spaced contiguous rows (batches folded)
-    if (!rows.fused || !rows.half || rows.d.nb != 1 || rows.d.in_es != 1 || rows.d.out_es != 1 ||
+    if (!rows.fused || rows.tile || !rows.half || rows.d.nb != 1 || rows.d.in_es != 1 || rows.d.out_es != 1 ||
         rows.d.in_ls != rows.n || rows.d.out_ls != rows.n || rows.expr.empty() || rows.expr.back() != '>')
         return DTFFT_HIP_SUCCESS;
     // cols: the fused column form reading the rows' output across lines: n lines side by side,
     // its FFT axis (nlc rows) n elements apart, batches of whole planes
     const int64_t n = rows.n, nlc = cols.n, B = cols.lpb;
     const r2r_desc_h& cd = cols.d;
-    if (!cols.fused || !cols.half || cols.dbl != rows.dbl || B <= 0 || n % B != 0 || cd.nl != n || cd.in_ls != 1 ||
+    if (!cols.fused || cols.tile || !cols.half || cols.dbl != rows.dbl || B <= 0 || n % B != 0 || cd.nl != n || cd.in_ls != 1 ||
         cd.in_es != n || cd.in_ts != 0 || (cd.nb > 1 && cd.in_bs != n * nlc) || rows.d.nl != nlc * cd.nb)
         return DTFFT_HIP_SUCCESS;
     if (rows.lpb <= 0 || nlc % rows.lpb != 0) return DTFFT_HIP_SUCCESS;  // row tiles within one batch
@@ -192,6 +271,10 @@ int32_t r2r_stage::init_cols(int kind_, int64_t n_, bool dbl_, int64_t nl, int64
     const size_t ec = dbl_ ? 16 : 8, er = dbl_ ? 8 : 4;
     const int lpb = (int)(128 / er);  // a tile row is one 128-byte piece of LPB reals
     if (nl % lpb != 0) return DTFFT_HIP_SUCCESS;
+    if ((n_ & (n_ - 1)) != 0) {  // as init: the general kernel is the faster one (384 points 291 against 367 us)
+        TRY(init_tile(kind_, n_, dbl_, nl, nb, 1, in_bs, in_es, out_ls, out_bs, out_es, ok));
+        if (*ok) return DTFFT_HIP_SUCCESS;
+    }
     const int64_t mf = n_ / 2;
     fft_config c = default_fft_config((int)mf, dbl_, false, false, 0, 0);
     c.radices = hrad;
@@ -212,7 +295,7 @@ int32_t r2r_stage::init_cols(int kind_, int64_t n_, bool dbl_, int64_t nl, int64
                     std::to_string(mf);
     for (int r : c.radices) e += ", " + std::to_string(r);
     e += ">, " + std::to_string(c.tpl) + ", " + std::to_string(c.lpb) + ", " + std::to_string(c.pad) + ", " +
-         std::to_string(kind) + ", true, true, true" + (out_cols ? ", true>" : ", false>");
+         std::to_string(kind) + ", true, true" + (out_cols ? ", true>" : ", false>");
     TRY(rtc_get("r2r", e, &fk));
     expr = e;
     this->lpb = c.lpb;
