@@ -196,10 +196,15 @@ static size_t lds_dma(const fft_config& c) {
     return (c.dma == 2 ? 1 : 2) * std::max(load, stage) + std::max<size_t>(1, tw) * 16;
 }
 
+// The LDS-DMA kernels hold radices up to 16: a large prime's butterfly needs bfly_large.
+static bool dma_radices(const fft_config& c) {
+    return std::all_of(c.radices.begin(), c.radices.end(), [](int r) { return r <= 16; });
+}
+
 // Whether a fused column-in C2R stage can use fft_c2r_dma_kernel.
 static bool c2r_dma_ok(const fft_config& c, const lines_desc& d) {
     const int64_t es = elem_bytes(c.dbl);
-    return c.kind == 2 && (c.dma == 1 || c.dma == 2) && c.n > 1 && c.n % 8 == 0 && c.lpb * es == 128 && (c.tpl * c.lpb) % 64 == 0 &&
+    return dma_radices(c) && c.kind == 2 && (c.dma == 1 || c.dma == 2) && c.n > 1 && c.n % 8 == 0 && c.lpb * es == 128 && (c.tpl * c.lpb) % 64 == 0 &&
            c.tpl * c.lpb <= 1024 && d.in_ls == 1 && d.out_ns == 1 && d.nl % c.lpb == 0 && (d.in_ns * es) % 16 == 0 &&
            (d.in_bs * es) % 16 == 0 && lds_dma(c) <= kMaxLds;
 }
@@ -209,7 +214,7 @@ bool dma_ok(const fft_config& c, const lines_desc& d) {
     const int64_t es = elem_bytes(c.dbl);
     const bool out_ok = c.out_cols ? (d.out_ls == 1 && (d.out_ns * es) % 16 == 0 && (d.out_bs * es) % 16 == 0)
                                    : d.out_ns == 1;
-    return c.kind == 0 && c.in_cols && c.seg == 0 && c.n > 1 && c.n % 8 == 0 && c.lpb * es == 128 &&
+    return dma_radices(c) && c.kind == 0 && c.in_cols && c.seg == 0 && c.n > 1 && c.n % 8 == 0 && c.lpb * es == 128 &&
            (c.tpl * c.lpb) % 64 == 0 && c.tpl * c.lpb <= 1024 && d.in_ls == 1 && out_ok && d.nl % c.lpb == 0 &&
            (d.in_ns * es) % 16 == 0 && (d.in_bs * es) % 16 == 0 && lds_dma(c) <= kMaxLds;
 }
@@ -857,7 +862,8 @@ int32_t plan_fft_stage(int n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, i
         // The radices as equal as they come, one butterfly per thread for powers of two from 256
         // on, else 32 threads (320 = 8 8 5: 181 us per GiB, 198 us on 64; 192 = 16 12: 176, 184 us
         // on 16).
-        if (factorize(n, c.radices)) {
+        if (factorize(n, rad)) {
+            c.radices = rad;
             const int t = n / *std::max_element(c.radices.begin(), c.radices.end());
             c.tpl = n >= 256 && (n & (n - 1)) == 0 ? t : n <= 512 ? 32 : 64;
         }
