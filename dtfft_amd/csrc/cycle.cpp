@@ -41,10 +41,11 @@ struct length_group {
     fft_config cfg;
     std::shared_ptr<twiddles> tw;
     const rtc_kernel* k = nullptr;
+    const rtc_kernel* k_alt = nullptr;  // cfg.dma: the plain column kernel, for misaligned buffers
     void* d_gs = nullptr;
     void* d_items = nullptr;
     int nitems = 0;
-    unsigned grid = 0, block = 0;
+    unsigned grid = 0, grid_alt = 0, block = 0;
     int64_t work = 0;  // elements moved, for ordering the launches
     ~length_group() {
         if (d_gs) hipFree(d_gs);
@@ -116,8 +117,24 @@ static std::string tile_type(const fft_config& c) {
 static int32_t launch_group(const length_group& grp, int inv, const void* in, void* out, hipStream_t st);
 
 static std::string group_expr(const fft_config& cf, bool dbl) {
+    if (cf.dma) {
+        std::string s = std::string("batched_cols_dma_kernel<") + (dbl ? "double" : "float") + ", dtfft::sched<" +
+                        std::to_string(cf.n);
+        for (int r : cf.radices) s += ", " + std::to_string(r);
+        return s + ">, " + std::to_string(cf.tpl) + ", " + std::to_string(cf.lpb) + ", " + std::to_string(cf.pad) +
+               (cf.out_cols ? ", true>" : ", false>");
+    }
     return std::string("batched_fft_kernel<") + (dbl ? "double" : "float") + ", " + std::to_string(cf.tpl * cf.lpb) +
            ", " + tile_type(cf) + ">";
+}
+
+// Resident blocks of k at the most, no more than there are work items.
+static unsigned resident_grid(const rtc_kernel* k, unsigned block, int nitems) {
+    int per_cu = 1;
+    if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k->fn, (int)block, 0) != hipSuccess || per_cu < 1)
+        per_cu = 1;
+    const int64_t resident = (int64_t)per_cu * std::max(1, device().num_cus);
+    return (unsigned)std::max<int64_t>(1, std::min<int64_t>(nitems, resident));
 }
 
 // One launch of a stage for the grids `members`, all of one axis length, with tile shape cf.
@@ -127,6 +144,11 @@ static int32_t make_group(const cycle_t* cy, const std::vector<stage_spec>& spec
     grp->cfg = cf;
     grp->block = (unsigned)(cf.tpl * cf.lpb);
     TRY(rtc_get("fft", group_expr(cf, cy->dbl), &grp->k));
+    if (cf.dma) {
+        fft_config alt = cf;
+        alt.dma = 0;
+        TRY(rtc_get("fft", group_expr(alt, cy->dbl), &grp->k_alt));
+    }
     TRY(get_twiddles(cf.n, cf.radices, cy->dbl, &grp->tw));
     std::vector<grid_stage_h> gs;
     std::vector<int> flat;
@@ -147,17 +169,30 @@ static int32_t make_group(const cycle_t* cy, const std::vector<stage_spec>& spec
     if (!compile_only()) {
         HIP_TRY(hipMalloc(&grp->d_gs, sizeof(grid_stage_h) * gs.size()));
         HIP_TRY(hipMemcpy(grp->d_gs, gs.data(), sizeof(grid_stage_h) * gs.size(), hipMemcpyHostToDevice));
-        HIP_TRY(hipMalloc(&grp->d_items, sizeof(int) * flat.size()));
-        HIP_TRY(hipMemcpy(grp->d_items, flat.data(), sizeof(int) * flat.size(), hipMemcpyHostToDevice));
-        int per_cu = 1;
-        if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, grp->k->fn, (int)grp->block, 0) !=
-                hipSuccess || per_cu < 1)
-            per_cu = 1;
-        const int64_t resident = (int64_t)per_cu * std::max(1, device().num_cus);
-        grp->grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(grp->nitems, resident));
+        grp->grid = resident_grid(grp->k, grp->block, grp->nitems);
+        if (grp->k_alt) grp->grid_alt = resident_grid(grp->k_alt, grp->block, grp->nitems);
+        // Blocks are dealt to the 8 XCDs in turn.  Column tiles whose row pieces straddle 128-byte
+        // lines share them with the next tile of their grid: in each round of blocks an XCD takes
+        // neighbouring items (the map of xcd_tile in device/fft.hip), so that they share an L2.
+        const int64_t es = cy->dbl ? 16 : 8, G = grp->grid, whole = G % 8 == 0 ? grp->nitems / G * G : 0;
+        bool near = false;
+        for (int g : members) near |= cf.in_cols && specs[g].in_ns * es % 128 != 0;
+        std::vector<int> order = flat;
+        for (int64_t i = 0; near && i < whole; i++) {
+            const int64_t b = i % G, t = i - b + (b % 8) * (G / 8) + b / 8;
+            order[2 * i] = flat[2 * t];
+            order[2 * i + 1] = flat[2 * t + 1];
+        }
+        HIP_TRY(hipMalloc(&grp->d_items, sizeof(int) * order.size()));
+        HIP_TRY(hipMemcpy(grp->d_items, order.data(), sizeof(int) * order.size(), hipMemcpyHostToDevice));
     }
     out = std::move(grp);
     return DTFFT_HIP_SUCCESS;
+}
+
+// Whether every row piece of the grid's tiles can be loaded into LDS directly.
+static bool grid_dma_ok(const fft_config& c, const stage_spec& q) {
+    return dma_ok(c, make_lines(q.nl, q.nb, q.in_ls, q.in_bs, q.in_ns, q.out_ls, q.out_bs, q.out_ns, c.lpb));
 }
 
 // Candidate tile shapes of a group for the autotuner, the default first: radix schedules of
@@ -199,7 +234,9 @@ static uint64_t fnv1a_ints(const std::vector<int64_t>& v) {
 // fastest (the project's replacement of dtfft_nvrtc_block_optimizer for the batched cycle).
 // The choice is stored as a tuning record keyed by the group's length, layout and lines.
 static int32_t tune_group(cycle_t* cy, const std::vector<stage_spec>& specs, const std::vector<int>& members,
-                          bool in_cols, bool out_cols, void* scratch_in, void* scratch_out, fft_config& best) {
+                          bool in_cols, bool out_cols, void* scratch_in, void* scratch_out, fft_config& best,
+                          bool& tuned) {
+    tuned = false;
     const int n = (int)specs[members[0]].n;
     std::vector<int64_t> sig;
     int64_t lines = 0;
@@ -215,18 +252,26 @@ static int32_t tune_group(cycle_t* cy, const std::vector<stage_spec>& specs, con
     best = default_fft_config(n, cy->dbl, in_cols, out_cols, lines, INT64_MAX);
     std::string rec;
     if (tune_lookup(key, rec)) {
-        int t, l, p;
+        int t, l, p, dm = 0;
         char rads[128] = {0};
         std::vector<int> r;
-        if (std::sscanf(rec.c_str(), "%d %d %d %127s", &t, &l, &p, rads) == 4 && parse_radices(rads, n, r)) {
+        // "tpl lpb pad radices dma" (records without the last field are of the plain kernel)
+        if (std::sscanf(rec.c_str(), "%d %d %d %127s %d", &t, &l, &p, rads, &dm) >= 4 && parse_radices(rads, n, r)) {
             fft_config c = best;
-            c.tpl = t; c.lpb = l; c.pad = p; c.radices = r;
-            if (t * l >= 1 && t * l <= 1024 && fft_lds_bytes(c) <= 160 * 1024) best = c;
+            c.tpl = t; c.lpb = l; c.pad = p; c.radices = r; c.dma = dm == 2 ? 2 : 0;
+            bool fits = t * l >= 1 && t * l <= 1024 && fft_lds_bytes(c) <= 160 * 1024;
+            if (c.dma) for (int g : members) fits = fits && grid_dma_ok(c, specs[g]);
+            if (fits) { best = c; tuned = true; }
         }
         return DTFFT_HIP_SUCCESS;
     }
     if (cy->effort < DTFFT_HIP_MEASURE || compile_only() || !scratch_in) return DTFFT_HIP_SUCCESS;
     auto cands = group_candidates(n, cy->dbl, in_cols, out_cols, lines, cy->effort);
+    if (in_cols && global_config().lds_dma != 0) {
+        const fft_config c = dma_config(best, 2);
+        if (std::all_of(members.begin(), members.end(), [&](int g) { return grid_dma_ok(c, specs[g]); }))
+            cands.push_back(c);
+    }
     // compile the candidates side by side (hipRTC programs are independent)
     {
         std::vector<std::thread> pool;
@@ -263,8 +308,9 @@ static int32_t tune_group(cycle_t* cy, const std::vector<stage_spec>& specs, con
     std::string r;
     for (size_t i = 0; i < best.radices.size(); i++) r += (i ? "," : "") + std::to_string(best.radices[i]);
     char buf[160];
-    std::snprintf(buf, sizeof buf, "%d %d %d %s", best.tpl, best.lpb, best.pad, r.c_str());
+    std::snprintf(buf, sizeof buf, "%d %d %d %s %d", best.tpl, best.lpb, best.pad, r.c_str(), best.dma);
     tune_store(key, buf);
+    tuned = true;
     return DTFFT_HIP_SUCCESS;
 }
 
@@ -294,10 +340,21 @@ static int32_t build_stage(cycle_t* cy, int dir, int s, void* scratch_in, void* 
         const bool in_cols = sp.in_ns != 1 && sp.in_ls == 1;
         const bool out_cols = sp.out_ns != 1 && sp.out_ls == 1;
         fft_config cf;
-        TRY(tune_group(cy, specs, members, in_cols, out_cols, scratch_in, scratch_out, cf));
-        std::unique_ptr<length_group> grp;
-        TRY(make_group(cy, specs, members, cf, grp));
-        groups.push_back(std::move(grp));
+        bool tuned = false;
+        TRY(tune_group(cy, specs, members, in_cols, out_cols, scratch_in, scratch_out, cf, tuned));
+        std::vector<int> direct;  // grids of the LDS-DMA launch
+        const fft_config cd = dma_config(cf, 2);
+        if (!tuned && in_cols && !cy->dbl && global_config().lds_dma != 0) {
+            for (int g : members) if (grid_dma_ok(cd, specs[g])) direct.push_back(g);
+            members.erase(std::remove_if(members.begin(), members.end(),
+                                         [&](int g) { return grid_dma_ok(cd, specs[g]); }), members.end());
+        }
+        for (const bool dma : {true, false}) {
+            if ((dma ? direct : members).empty()) continue;
+            std::unique_ptr<length_group> grp;
+            TRY(make_group(cy, specs, dma ? direct : members, dma ? cd : cf, grp));
+            groups.push_back(std::move(grp));
+        }
     }
     std::stable_sort(groups.begin(), groups.end(),
                      [](const std::unique_ptr<length_group>& a, const std::unique_ptr<length_group>& b) {
@@ -316,6 +373,8 @@ static int32_t launch_group(const length_group& grp, int inv, const void* in, vo
     void* itp = grp.d_items;
     int nitems = grp.nitems;
     void* args[] = {(void*)&in, &out, &gsp, &itp, &nitems, &inv};
+    if (grp.cfg.dma && (((uintptr_t)in % 16) != 0 || ((uintptr_t)out % 16) != 0))
+        return launch(grp.k_alt, grp.grid_alt, grp.block, st, args);
     return launch(grp.k, grp.grid, grp.block, st, args);
 }
 

@@ -979,9 +979,10 @@ __global__ void gen_rtwiddles_f64(cx<double>* tw, int off, int n, int cnt) {
 // then writes the load layout back and the store mirrors the load, 16 bytes per lane.
 // Barriers inside a tile synchronise LDS only (lgkmcnt), so the next tile's loads stay in
 // flight; they are waited for at the top of the next tile.  Twiddles live in LDS (no global
-// loads other than the tile loads).  The host uses this kernel only when nl % LPB == 0,
-// N % 8 == 0, in_ls == 1, out_ns == 1 (out_ls == 1 for OUT_COLS) and every row segment is
-// 16-byte aligned.
+// loads other than the tile loads).  A batch's last tile may hold fewer lines: the lanes past
+// them load and store nothing, and the passes transform whatever the buffer holds there.  The
+// host uses this kernel only when in_ls == 1, out_ns == 1 (out_ls == 1 for OUT_COLS) and every
+// row segment starts and ends on 16 bytes.
 // ---------------------------------------------------------------------------
 #ifndef DTFFT_LDS_BARRIER
 #define DTFFT_LDS_BARRIER() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
@@ -1013,36 +1014,49 @@ struct cols_dma {
     static_assert(LPB * ES == 128, "a tile row is one 128-byte segment");
     static constexpr int N = S::N;
     static constexpr int NP = S::NP;
-    static_assert(N % 8 == 0 && NP > 0, "rows come in groups of 8");
+    static_assert(NP > 0, "a length-1 line is a copy");
     static constexpr int NT = TPL * LPB;
     static_assert(NT % 64 == 0, "whole waves");
     static constexpr int NW = NT / 64;
     static constexpr int GROUPB = 1024 + 128;
-    static constexpr int NG = N / 8;
+    static constexpr int NG = (N + 7) / 8;
     static constexpr int LD = (N + PAD) | 1;
-    static constexpr int LOADB = NG * GROUPB;
+    // the last group needs no padding after its rows
+    static constexpr int LOADB = (NG - 1) * GROUPB + (N - 8 * (NG - 1)) * 128;
     static constexpr int STAGEB = LPB * LD * ES;
     static constexpr int BUFE = (LOADB > STAGEB ? LOADB : STAGEB) / ES;
     static constexpr int TWN = S::TW_SIZE > 0 ? S::TW_SIZE : 1;
-
     // element index of (n, line) in the load layout
     static __device__ __forceinline__ int a_off(int n, int line) {
         return (n >> 3) * (GROUPB / ES) + (n & 7) * (128 / ES) + line;
     }
 
-    static __device__ __forceinline__ void bases(const lines_desc& d, i64 t, i64& ibase, i64& obase) {
+    static constexpr int PER = 16 / ES;  // complex values per 16-byte chunk
+
+    // element offsets of tile t and its lines
+    static __device__ __forceinline__ int bases(const lines_desc& d, i64 t, i64& ibase, i64& obase) {
         const i64 tl = t % d.ntl, b = t / d.ntl;
         ibase = tl * (d.in_ts ? d.in_ts : (i64)LPB) + b * d.in_bs;
         obase = tl * LPB * d.out_ls + b * d.out_bs;
+        const i64 left = d.nl - tl * LPB;
+        return left < LPB ? (int)left : LPB;
     }
 
-    // this wave's share of the loads of the tile at ibase into buf
-    static __device__ __forceinline__ void load(const cx<T>* in, cx<T>* buf, const lines_desc& d, i64 ibase) {
+    // this wave's share of the loads of tile t into buf
+    static __device__ __forceinline__ void load(const cx<T>* in, cx<T>* buf, const lines_desc& d, i64 t) {
         const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
         const int row = lane >> 3, chunk = lane & 7;
-        for (int q = wave; q < NG; q += NW) {
-            const char* g = (const char*)(in + ibase + (i64)(q * 8 + row) * d.in_ns) + chunk * 16;
-            DTFFT_LOAD_LDS16(g, (char*)buf + q * GROUPB);
+        i64 ibase, obase;
+        const int lines = bases(d, t, ibase, obase);
+        // lanes past the tile's last line start past its last row
+        const int r0 = lines == LPB || chunk * PER < lines ? row : N;
+        const char* g0 = (const char*)(in + ibase) + chunk * 16;
+        if (N % 8 == 0 && lines == LPB) {
+            for (int q = wave; q < NG; q += NW)
+                DTFFT_LOAD_LDS16(g0 + (i64)(q * 8 + row) * d.in_ns * ES, (char*)buf + q * GROUPB);
+        } else {
+            for (int q = wave; q < NG; q += NW)
+                if (q * 8 + r0 < N) DTFFT_LOAD_LDS16(g0 + (i64)(q * 8 + row) * d.in_ns * ES, (char*)buf + q * GROUPB);
         }
     }
 
@@ -1112,13 +1126,14 @@ struct cols_dma {
     static __device__ __forceinline__ void store(const cx<T>* buf, cx<T>* out, const lines_desc& d, i64 t,
                                                  bool inv) {
         i64 ibase, obase;
-        bases(d, t, ibase, obase);
+        const int lines = bases(d, t, ibase, obase);
         if constexpr (OUT_COLS) {
             // mirror of load(): lane l of group q stores bytes 16 l .. 16 l + 15 of the group
             const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
             const int row = lane >> 3, chunk = lane & 7;
-            constexpr int PER = 16 / ES;  // complex values per 16-byte chunk
+            const int r0 = lines == LPB || chunk * PER < lines ? row : N;
             for (int q = wave; q < NG; q += NW) {
+                if ((N % 8 != 0 || lines != LPB) && q * 8 + r0 >= N) continue;
                 const cx<T>* src = buf + q * (GROUPB / ES) + row * (128 / ES) + chunk * PER;
                 cx<T>* dst = out + obase + (i64)(q * 8 + row) * d.out_ns + chunk * PER;
 #pragma unroll
@@ -1131,11 +1146,17 @@ struct cols_dma {
         } else {
             const int line = threadIdx.x / TPL, j = threadIdx.x % TPL;
             cx<T>* o = out + obase + (i64)line * d.out_ls;
+            if (line < lines) {
 #pragma unroll 4
-            for (int n = j; n < N; n += TPL) {
-                cx<T> y = buf[line * LD + n];
-                if (inv) y = conj(y);
-                store_nt(&o[n], y);
+                for (int n = j; n < N; n += TPL) {
+                    cx<T> y = buf[line * LD + n];
+                    if (inv) y = conj(y);
+                    // Rows that end inside a 128-byte line share it with their neighbours: plain
+                    // stores, which meet in the L2 (us per 2 GiB at 36, 100 and 210 points:
+                    // non-temporal 550, 408 and 461, plain 384, 378 and 380).
+                    if constexpr (N * ES % 128 == 0) store_nt(&o[n], y);
+                    else o[n] = y;
+                }
             }
         }
     }
@@ -1155,12 +1176,12 @@ fft_cols_dma_kernel(const cx<T>* __restrict__ in, cx<T>* __restrict__ out,
     for (int i = threadIdx.x; i < S::TW_SIZE; i += K::NT) twl[i] = tw[i];
     const bool iv = inv != 0;
     const i64 G = gridDim.x;
-    i64 t = blockIdx.x, ib, ob;
-    if (t < d.ntiles) { K::bases(d, t, ib, ob); K::load(in, buf_a, d, ib); }
+    i64 t = blockIdx.x;
+    if (t < d.ntiles) K::load(in, buf_a, d, t);
     DTFFT_WAIT_ALL();
     __syncthreads();  // first tile and twiddles in LDS
     i64 tn = t + G;
-    if (tn < d.ntiles) { K::bases(d, tn, ib, ob); K::load(in, buf_b, d, ib); }
+    if (tn < d.ntiles) K::load(in, buf_b, d, tn);
     // Three stages in flight: the passes of tile t run while the next tile's loads and the
     // previous tile's stores are outstanding.  The one wait per tile (for everything issued,
     // since loads and stores share one counter) comes after the passes, when both were issued
@@ -1173,7 +1194,7 @@ fft_cols_dma_kernel(const cx<T>* __restrict__ in, cx<T>* __restrict__ out,
         K::store(buf_a, out, d, t, iv);
         DTFFT_LDS_BARRIER();  // every wave has read its part of buf_a
         i64 tnn = tn + G;
-        if (tnn < d.ntiles) { K::bases(d, tnn, ib, ob); K::load(in, buf_a, d, ib); }
+        if (tnn < d.ntiles) K::load(in, buf_a, d, tnn);
         t = tn;
         tn = tnn;
         if (t >= d.ntiles) break;
@@ -1183,14 +1204,14 @@ fft_cols_dma_kernel(const cx<T>* __restrict__ in, cx<T>* __restrict__ out,
         K::store(buf_b, out, d, t, iv);
         DTFFT_LDS_BARRIER();
         tnn = tn + G;
-        if (tnn < d.ntiles) { K::bases(d, tnn, ib, ob); K::load(in, buf_b, d, ib); }
+        if (tnn < d.ntiles) K::load(in, buf_b, d, tnn);
         t = tn;
         tn = tnn;
     }
 }
 
-// Single-buffer variant: one tile buffer per block (about half the LDS), so that two blocks
-// share a CU and overlap each other's loads with their passes and stores.
+// Single-buffer variant: one tile buffer per block (about half the LDS), so that two blocks and
+// more share a CU and overlap each other's loads with their passes and stores.
 template <typename T, class S, int TPL, int LPB, int PAD, bool OUT_COLS = false>
 __global__ void __launch_bounds__(TPL * LPB)
 fft_cols_dma1_kernel(const cx<T>* __restrict__ in, cx<T>* __restrict__ out,
@@ -1198,16 +1219,49 @@ fft_cols_dma1_kernel(const cx<T>* __restrict__ in, cx<T>* __restrict__ out,
     typedef dtfft::cols_dma<T, S, TPL, LPB, PAD, OUT_COLS> K;
     __shared__ cx<T> buf[K::BUFE];
     __shared__ typename tw_of<T>::type twl[K::TWN];
-    for (int i = threadIdx.x; i < S::TW_SIZE; i += K::NT) twl[i] = tw[i];
     const bool iv = inv != 0;
-    for (i64 t = blockIdx.x; t < d.ntiles; t += gridDim.x) {
-        i64 ib, ob;
-        K::bases(d, t, ib, ob);
-        K::load(in, buf, d, ib);
+    const i64 G = gridDim.x;
+    // Row pieces that straddle 128-byte lines share them with the neighbouring tiles: those on one
+    // XCD, as in fft_c2c_kernel.  Whole lines are gathered in tile order.
+    const bool near = d.in_ns * K::ES % 128 != 0;
+    const i64 slots = near ? (d.ntiles + G - 1) / G * G : d.ntiles;
+    for (i64 s = blockIdx.x; s < slots; s += G) {
+        const i64 t = near ? dtfft::xcd_tile(s, G) : s;
+        if (t >= d.ntiles) continue;
+        K::load(in, buf, d, t);
+        for (int i = threadIdx.x; i < S::TW_SIZE; i += K::NT) twl[i] = tw[i];
         DTFFT_WAIT_ALL();
         __syncthreads();
         K::tile(buf, out, twl, d, t, iv);
         __syncthreads();  // the staged rows are read before the next tile's loads land
+    }
+}
+
+// The same on the work items of batched_fft_kernel: persistent blocks, one tile buffer each.  64
+// grids of 48 to 384 points an axis, FP32: the forward and backward cycle 5550 -> 5430 us.
+template <typename T, class S, int TPL, int LPB, int PAD, bool OUT_COLS>
+__global__ void __launch_bounds__(TPL * LPB)
+batched_cols_dma_kernel(const cx<T>* __restrict__ in, cx<T>* __restrict__ out,
+                        const dtfft::grid_stage* __restrict__ gs, const int2* __restrict__ items, int nitems,
+                        int inv) {
+    typedef dtfft::cols_dma<T, S, TPL, LPB, PAD, OUT_COLS> K;
+    typedef typename tw_of<T>::type tw_t;
+    __shared__ cx<T> buf[K::BUFE];
+    __shared__ tw_t twl[K::TWN];
+    for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
+        const int2 w = items[it];
+        const dtfft::grid_stage& g = gs[w.x];
+        const dtfft::lines_desc d = g.d;
+        K::load(in + g.in_off, buf, d, w.y);
+        if (it == (int)blockIdx.x) {
+            // every grid of the launch has the same length, so the same table
+            const tw_t* tw = (const tw_t*)g.tw;
+            for (int i = threadIdx.x; i < S::TW_SIZE; i += K::NT) twl[i] = tw[i];
+        }
+        DTFFT_WAIT_ALL();
+        __syncthreads();
+        K::tile(buf, out + g.out_off, twl, d, w.y, inv != 0);
+        __syncthreads();  // the tile is read before the next one's loads land
     }
 }
 

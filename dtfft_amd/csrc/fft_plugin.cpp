@@ -189,7 +189,8 @@ static size_t lds_dma(const fft_config& c) {
         if (c.dma == 1) return 2 * std::max(load, stage) + twb + (size_t)(c.n / 2 + 1) * 16 + 16;
         return std::max(load, stage) + (c.twl ? twb : 0);
     }
-    const size_t load = (size_t)(c.n / 8) * 1152;
+    const size_t groups = (size_t)((c.n + 7) / 8);
+    const size_t load = (groups - 1) * 1152 + ((size_t)c.n - 8 * (groups - 1)) * 128;
     const size_t stage = (size_t)c.lpb * (size_t)((c.n + c.pad) | 1) * es;
     size_t tw = 0, L = 1;
     for (int r : c.radices) { tw += L * (size_t)(r - 1); L *= (size_t)r; }
@@ -214,8 +215,8 @@ bool dma_ok(const fft_config& c, const lines_desc& d) {
     const int64_t es = elem_bytes(c.dbl);
     const bool out_ok = c.out_cols ? (d.out_ls == 1 && (d.out_ns * es) % 16 == 0 && (d.out_bs * es) % 16 == 0)
                                    : d.out_ns == 1;
-    return dma_radices(c) && c.kind == 0 && c.in_cols && c.seg == 0 && c.n > 1 && c.n % 8 == 0 && c.lpb * es == 128 &&
-           (c.tpl * c.lpb) % 64 == 0 && c.tpl * c.lpb <= 1024 && d.in_ls == 1 && out_ok && d.nl % c.lpb == 0 &&
+    return dma_radices(c) && c.kind == 0 && c.in_cols && c.seg == 0 && c.n > 1 && c.lpb * es == 128 &&
+           (c.tpl * c.lpb) % 64 == 0 && c.tpl * c.lpb <= 1024 && d.in_ls == 1 && out_ok && (d.nl * es) % 16 == 0 &&
            (d.in_ns * es) % 16 == 0 && (d.in_bs * es) % 16 == 0 && lds_dma(c) <= kMaxLds;
 }
 
@@ -753,6 +754,34 @@ static int64_t span(const lines_desc& d, bool in, int n) {
     return (d.nl - 1) * ls + (d.nb - 1) * bs + (int64_t)(n - 1) * ns + 1;
 }
 
+// The shape of an LDS-DMA column stage for the lines of cfg: the radices as equal as they come.
+// Single buffer (dma 2): several blocks share a CU, 16 threads per line up to 255 points, 32 up to
+// 512 (us per 2 GiB: 160 points 360 on 16, 394 on 20; 96 points 348 on 16, 389 on 12; 320 points 362
+// on 32, 389 on 16; 512 points 384 on 32, 392 on 64), but half of that where a pass would hold more
+// than 16 points in a thread: over 128 VGPRs only one block of 512 threads fits a CU (480 = 10 8 6:
+// 539 on 32, 420 on 16; 900 = 10 10 9: 829 on 64, 536 on 32).  Double buffer (dma 1, one block per CU):
+// one butterfly per thread for powers of two from 256 on, else 32 threads.
+fft_config dma_config(const fft_config& cfg, int dma) {
+    fft_config c = cfg;
+    c.dma = dma;
+    c.staged = false;
+    c.lpb = 128 / elem_bytes(c.dbl);  // a tile row is one 128-byte piece
+    std::vector<int> rad;
+    if (factorize(c.n, rad)) {
+        c.radices = rad;
+        if (dma == 2) {
+            c.tpl = c.n <= 32 ? 8 : c.n < 256 ? 16 : c.n <= 512 ? 32 : 64;
+            int points = 0;  // of one thread in the pass that holds most
+            for (int r : rad) points = std::max(points, (c.n / r + c.tpl - 1) / c.tpl * r);
+            if (c.tpl > 16 && points > 16) c.tpl /= 2;
+        } else {
+            c.tpl = c.n <= 512 ? 32 : 64;
+            if (c.n >= 256 && (c.n & (c.n - 1)) == 0) c.tpl = c.n / rad[0];
+        }
+    }
+    return c;
+}
+
 int32_t plan_fft_stage(int n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, int64_t in_bs, int64_t in_ns,
                        int64_t out_ls, int64_t out_bs, int64_t out_ns, bool inplace, int effort,
                        hipStream_t stream, fft_stage* st, int lds_dma) {
@@ -849,25 +878,16 @@ int32_t plan_fft_stage(int n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, i
     if (lds_dma == 0) {
         cfg.dma = 0;
     } else if (!cfg.dma && (lds_dma >= 2 || (!tuned && !dbl))) {
-        // Default for FP32 column-in passes: the LDS-DMA kernels measured 10-14 % faster than
-        // the plain column kernel on MI355X.  512^3 column-in / row-out pass: 431 us with one
-        // tile per block, 444 us persistent with two buffers, 498 us plain.  The in-place
-        // column pass runs best persistent with two buffers and half the threads per line:
-        // 444 us, against 475 us with one tile per block and 495 us plain.  FP64 keeps the
-        // plain kernel, which the autotuner preferred there.
-        fft_config c = cfg;
-        c.dma = lds_dma == 2 ? 1 : lds_dma == 3 ? 2 : (c.out_cols ? 1 : 2);
-        c.staged = false;
-        c.lpb = 128 / elem_bytes(dbl);  // a tile row is one 128-byte piece
-        // The radices as equal as they come, one butterfly per thread for powers of two from 256
-        // on, else 32 threads (320 = 8 8 5: 181 us per GiB, 198 us on 64; 192 = 16 12: 176, 184 us
-        // on 16).
-        if (factorize(n, rad)) {
-            c.radices = rad;
-            const int t = n / *std::max_element(c.radices.begin(), c.radices.end());
-            c.tpl = n >= 256 && (n & (n - 1)) == 0 ? t : n <= 512 ? 32 : 64;
-        }
-        if (c.out_cols && lds_dma < 2 && n >= 256 && (n & (n - 1)) == 0) c.tpl = std::max(1, c.tpl / 2);
+        // Default for FP32 column-in passes, us per 2 GiB, LDS-DMA (one tile per block) against the
+        // plain column kernel: 16 points 354 / 404, 36 points 384 / 550, 64 points 346 / 395, 210
+        // points 380 / 490, 320 points 374 / 500, 512 points 384 / 442, 900 points 536 / 662; rows
+        // of 210 lines, whose pieces straddle 128-byte lines: 64 points 357 / 441, 320 points 419 /
+        // 514, 512 points 461 / 536.  In place from 48 points on (60 points 394 / 453, 36 points 467 /
+        // 408, 512 points 395 / 453).  Launches of few tiles are bound by latency, where the plain
+        // kernel's loads go straight to the first pass (256 points, 4 MB: 5.9 / 5.2).  FP64 keeps
+        // the plain kernel, which the autotuner preferred there.
+        fft_config c = dma_config(cfg, lds_dma == 2 ? 1 : 2);
+        const bool use = lds_dma >= 2 || (nl * nb >= 8192 && n >= (c.out_cols ? 48 : 16));
         bool wide = false;
         if (lds_dma == 1 && !dbl && inplace && cfg.out_cols && n >= 512) {
             // In-place FP32 column passes of n >= 512 where a 32-line tile (256-byte pieces of
@@ -885,7 +905,7 @@ int32_t plan_fft_stage(int n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, i
             apply_twl(w, d, 1);  // the measured form: persistent with LDS twiddles (>= 2048 tiles)
             if (w.twl && valid(w)) { cfg = w; rec_twl = -1; wide = true; }
         }
-        if (!wide && dma_ok(c, d)) { cfg = c; rec_twl = -1; }
+        if (!wide && use && dma_ok(c, d)) { cfg = c; rec_twl = -1; }
     }
     // persistent blocks with the twiddle table in LDS: as the tuning record says (the form it
     // was timed in), else by the rule of the configuration

@@ -167,6 +167,7 @@ struct fft_stage {
     int32_t run(const void* in, void* out, int sign, hipStream_t s) const;
 };
 // Whether a column-in / row-out stage can use fft_cols_dma_kernel (shape, strides, LDS).
+fft_config dma_config(const fft_config& cfg, int dma);
 bool dma_ok(const fft_config& c, const lines_desc& d);
 lines_desc make_lines(int64_t nl, int64_t nb, int64_t in_ls, int64_t in_bs, int64_t in_ns,
                       int64_t out_ls, int64_t out_bs, int64_t out_ns, int lpb);

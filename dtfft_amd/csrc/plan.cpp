@@ -147,7 +147,7 @@ static int32_t blocked_pair(plan_t* p, const fft_stage& rows, const fft_stage& c
         while (cc.lpb > 8 && cols.d.nl % cc.lpb != 0) cc.lpb /= 2;
         if (!p->dbl && cc.lpb < 16 && cc.tpl * 16 <= 1024) {
             cc.lpb = 16;
-            if (fft_lds_bytes(cc) > 64 * 1024) cc.lpb = 8;
+            if (fft_lds_bytes(cc) > 80 * 1024) cc.lpb = 8;
         }
     }
     if (!p->dbl && cc.lpb % 16 != 0) return DTFFT_HIP_SUCCESS;
@@ -173,8 +173,7 @@ static int32_t blocked_pair(plan_t* p, const fft_stage& rows, const fft_stage& c
     // other way round.  Under the default rule (lds_dma 1) the blocked stage takes it.
     fft_config c = cc;
     if (c.dma == 2 && p->lds_dma == 1) {
-        fft_config c2 = c;
-        c2.dma = 1;
+        const fft_config c2 = dma_config(c, 1);
         if (dma_ok(c2, bd)) c = c2;
     }
     TRY(rows_blk->init(r, rd));
@@ -213,8 +212,7 @@ static int32_t blocked_r2c(plan_t* p, bool* ok) {
     fft_config c = cc;
     // the persistent double-buffer LDS-DMA kernel is the faster form on a blocked input
     if (c.dma == 2 && p->lds_dma == 1) {
-        fft_config c2 = c;
-        c2.dma = 1;
+        const fft_config c2 = dma_config(c, 1);
         if (dma_ok(c2, bd)) c = c2;
     }
     if (c.dma && !dma_ok(c, bd)) return DTFFT_HIP_SUCCESS;
