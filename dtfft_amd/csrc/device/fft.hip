@@ -465,7 +465,7 @@ struct fft_tile {
     // Runs passes p..NP-1.  FIRST_G: pass 0 reads global (else LDS was filled and synced by
     // the caller).  LAST_G: the last pass writes global (else it leaves the line in LDS;
     // the caller syncs before reading it).
-    template <int p, bool FIRST_G, bool LAST_G>
+    template <int p, bool FIRST_G, bool LAST_G, int END = NP>
     static __device__ __forceinline__ void passes(const cx<T>* __restrict__ gin, cx<T>* __restrict__ gout,
                                                   const tw_t* __restrict__ tw, cx<T>* lds, i64 ibase,
                                                   i64 obase, const lines_desc& d, i64 l0, bool inv) {
@@ -482,7 +482,7 @@ struct fft_tile {
                 }
             }
         }
-        if constexpr (p < NP) {
+        if constexpr (p < END) {
             constexpr bool first = (p == 0);
             constexpr bool last = (p == NP - 1);
             if constexpr (first && FIRST_G && last) {
@@ -509,7 +509,7 @@ struct fft_tile {
                 __syncthreads();
                 pass<p, false, false, false>(gin, gout, tw, lds, ibase, obase, d, l0, inv);
             }
-            passes<p + 1, FIRST_G, LAST_G>(gin, gout, tw, lds, ibase, obase, d, l0, inv);
+            passes<p + 1, FIRST_G, LAST_G, END>(gin, gout, tw, lds, ibase, obase, d, l0, inv);
         }
     }
 
@@ -725,6 +725,93 @@ fft_c2c_kernel(const cx<T>* __restrict__ in, cx<T>* __restrict__ out,
     }
 }
 
+// The mirror pairs (k, M - k) that untangling works on, in registers.  A pass of radix R has NB = M / R
+// butterflies; b holds the elements b + r NB (inputs of the first pass, outputs of the last one),
+// and the mirror of b + s NB is (NB - b) + (R - 1 - s) NB, an element of butterfly NB - b.  So a
+// thread that takes both (unit u: b = u and NB - u) has R whole pairs.  Unit 0 takes butterfly 0,
+// which mirrors onto itself (element 0 onto M), and NB / 2 where NB is even: its slots are the pairs
+// of the first, then those of the second, and element M / 2, its own mirror, is left over.
+namespace dtfft {
+template <typename T, class S, int R>
+struct mirror_pairs {
+    typedef typename tw_of<T>::type tw_t;
+    static constexpr int M = S::N, NB = M / R;
+    static constexpr int UNITS = (NB + 1) / 2;
+    static constexpr bool EVEN = NB % 2 == 0;  // unit 0 has a second butterfly
+    static constexpr int H0 = (R + 1) / 2;     // unit 0: slots of butterfly 0
+
+    static __device__ __forceinline__ int second(int u) { return u ? NB - u : EVEN ? NB / 2 : 0; }
+    // element k of slot s (its mirror is M - k)
+    static __device__ __forceinline__ int elem(int u, int s) {
+        return u == 0 && s >= H0 ? NB / 2 + (s - H0) * NB : u + s * NB;
+    }
+    static __device__ __forceinline__ bool has(int u, int s) { return u != 0 || EVEN || s < H0; }
+    static __device__ __forceinline__ cx<T> sel(bool z, cx<T> a, cx<T> b) { return mk(z ? a.x : b.x, z ? a.y : b.y); }
+
+    // R2C: X_k and X_{M-k} of every pair from the outputs Z of butterflies u (v0) and second(u)
+    // (v1), as put(k, X).  With e = Z_k + conj Z_{M-k} and w = W^k (Z_k - conj Z_{M-k}):
+    // X_k = (e - i w) / 2 and, as W^{M-k} = -conj W^k, X_{M-k} = conj(e + i w) / 2.
+    template <class Put>
+    static __device__ __forceinline__ void untangle(int u, const cx<T>* v0, const cx<T>* v1, const tw_t* rtw,
+                                                    const Put& put) {
+        const bool z = u == 0;
+        const T half = (T)0.5;
+#pragma unroll
+        for (int s = 0; s < R; s++) {
+            cx<T> a, b;
+            if (s < H0) {
+                a = v0[s];
+                b = sel(z, v0[(R - s) % R], v1[R - 1 - s]);
+            } else {
+                a = sel(z, v1[s - H0], v0[s]);
+                b = sel(z, v1[R - 1 - (s - H0)], v1[R - 1 - s]);
+            }
+            if (has(u, s)) {
+                const int k = elem(u, s);
+                b = conj(b);
+                const cx<T> e = a + b, w = twmul(a - b, rtw[k]);
+                put(k, mk(half * (e.x + w.y), half * (e.y - w.x)));
+                put(M - k, mk(half * (e.x - w.y), half * (-e.y - w.x)));
+            }
+        }
+        if (M % 2 == 0 && z) put(M / 2, conj(R % 2 == 0 ? v0[R / 2] : v1[R / 2]));  // W^{M/2} = -i
+    }
+
+    // C2R: conj Z of the inputs of butterflies u and second(u) from X, get(k) = X_k:
+    // Z_k = e + i o with e = X_k + conj X_{M-k}, o = (X_k - conj X_{M-k}) conj(W^k), and
+    // Z_{M-k} = conj e + i conj o.
+    template <class Get>
+    static __device__ __forceinline__ void fold(int u, cx<T>* v0, cx<T>* v1, const tw_t* rtw, const Get& get) {
+        const bool z = u == 0;
+        cx<T> ck[R], cm[R], mid = mk((T)0, (T)0);
+#pragma unroll
+        for (int s = 0; s < R; s++) {
+            const int k = has(u, s) ? elem(u, s) : 0;
+            ck[s] = get(k);
+            cm[s] = get(M - k);
+        }
+        if (M % 2 == 0 && z) mid = get(M / 2);
+#pragma unroll
+        for (int s = 0; s < R; s++) {
+            const int k = has(u, s) ? elem(u, s) : 0;
+            cx<T> a = ck[s], b = cm[s];
+            if (s == 0 && z) { a.y = (T)0; b.y = (T)0; }  // Im X_0, Im X_M do not contribute
+            b = conj(b);
+            const cx<T> e = a + b, o = twmul(a - b, conj_tw(rtw[k]));
+            ck[s] = mk(e.x - o.y, -e.y - o.x);
+            cm[s] = mk(e.x + o.y, e.y - o.x);
+        }
+        mid = mid + mid;  // Z_{M/2} = 2 conj X_{M/2}
+#pragma unroll
+        for (int s = 0; s < R; s++) {
+            if (s < H0) v0[s] = ck[s];
+            else v0[s] = sel(z, (R % 2 == 0 && s == R / 2) ? mid : cm[R - s], ck[s]);
+            v1[s] = sel(z, s < R / 2 ? ck[H0 + s] : (R % 2 == 1 && s == R / 2) ? mid : cm[H0 + (R - 1 - s)], cm[R - 1 - s]);
+        }
+    }
+};
+}  // namespace dtfft
+
 // Real-to-complex along contiguous lines of even length n = 2M (rows layout).
 // The line is read as M complex values z_k = x_2k + i x_2k+1, transformed with the
 // M-point schedule S, and untangled:
@@ -736,39 +823,76 @@ fft_c2c_kernel(const cx<T>* __restrict__ in, cx<T>* __restrict__ out,
 template <typename T, class S, int TPL, int LPB, int PAD, int OSEG = 0>
 __global__ void __launch_bounds__(TPL * LPB)
 fft_r2c_kernel(const cx<T>* __restrict__ in, cx<T>* __restrict__ out,
-               const typename tw_of<T>::type* __restrict__ tw,
-               const typename tw_of<T>::type* __restrict__ rtw, dtfft::lines_desc d) {
+               const typename tw_of<T>::type* __restrict__ tw_,
+               const typename tw_of<T>::type* __restrict__ rtw_, dtfft::lines_desc d) {
     typedef dtfft::fft_tile<T, S, TPL, LPB, false, false, PAD, 0, OSEG> F;
     constexpr int M = S::N;
     __shared__ cx<T> lds[F::LDS_ELEMS];
     for (i64 t = blockIdx.x; t < d.ntiles; t += gridDim.x) {
         i64 l0, ibase, obase;
         F::tile_bases(d, t, l0, ibase, obase);
-        F::template passes<0, true, false>(in, out, tw, lds, ibase, obase, d, l0, false);
-        __syncthreads();
-        const T half = (T)0.5;
-        auto untangle = [&](int line, int k) {
-            const cx<T> a = lds[line * F::LD + F::lidx(k == M ? 0 : k)];
-            const cx<T> b = conj(lds[line * F::LD + F::lidx(k == 0 ? 0 : M - k)]);
-            const cx<T> s = a + b, df = a - b;
-            const cx<T> w = twmul(df, rtw[k]);                            // W^k (Z_k - conj Z_{M-k})
-            const cx<T> x = mk(half * (s.x + w.y), half * (s.y - w.x));  // (s - i w) / 2
-            // non-temporal (measured on MI355X, 1024 x 512 x 256 FP64 R2C rows: 394 against
-            // 399-403 us; FP32 unchanged within the noise)
-            store_nt(&out[obase + (i64)line * d.out_ls + F::out_elem(k, d)], x);
-        };
-        // LPB * M items, fully unrolled; the thread of k = 0 also writes X_M, so the loop has
-        // no mostly idle last round (measured on MI355X, 1024 x 512 x 256: FP32 rows 239
-        // against 254 us, FP64 380 against 397 us for a loop over LPB * (M + 1) items)
-        constexpr int UIT = (LPB * M + F::NT - 1) / F::NT;
+        const auto* tw = fresh(tw_);
+        const auto* rtw = fresh(rtw_);
+        if constexpr (F::NP > 1 && S::radix(F::NP - 1) <= 16) {
+            // the last pass and the untangling on mirror pairs in registers
+            // Chunked rows whose waves write runs of 512 bytes and more are stored non-temporal: they
+            // leave the caches to the pass that reads them (1024 x 512 x 256 FP32 forward and backward
+            // 1343 against 1305 us).  Shorter runs are whole 128-byte lines only in the L2 (128 points:
+            // 203 us per GiB, non-temporal 377).
+            constexpr bool NT = OSEG > 0 && TPL * (int)sizeof(cx<T>) >= 512;
+            constexpr int p = F::NP - 1, R = S::radix(p), TWO = S::tw_off(p);
+            typedef dtfft::mirror_pairs<T, S, R> P;
+            F::template passes<0, true, false, p>(in, out, tw, lds, ibase, obase, d, l0, false);
+            __syncthreads();
+            const int line = threadIdx.x / TPL, j = threadIdx.x % TPL;
+            cx<T>* o = out + obase + (i64)line * d.out_ls;
+            const bool live = l0 + line < d.nl;
+#pragma unroll 1
+            for (int u = j; u < P::UNITS; u += TPL) {
+                cx<T> v[2][R];
 #pragma unroll
-        for (int q = 0; q < UIT; q++) {
-            const int e = (int)threadIdx.x + q * F::NT;
-            if (UIT * F::NT == LPB * M || e < LPB * M) {
-                const int line = e / M, k = e % M;
-                if (l0 + line < d.nl) {
-                    untangle(line, k);
-                    if (k == 0) untangle(line, M);
+                for (int q = 0; q < 2; q++) {
+                    const int b = q ? P::second(u) : u;
+#pragma unroll
+                    for (int r = 0; r < R; r++) v[q][r] = lds[line * F::LD + F::lidx(b + r * P::NB)];
+#pragma unroll
+                    for (int r = 1; r < R; r++) v[q][r] = twmul(v[q][r], tw[TWO + b * (R - 1) + (r - 1)]);
+                    dtfft::bfly<T, R>::run(v[q]);
+                    __builtin_amdgcn_sched_barrier(0);  // one butterfly's twiddles at a time
+                }
+                P::untangle(u, v[0], v[1], rtw, [&](int k, cx<T> x) {
+                    if (!live) return;
+                    if constexpr (NT) store_nt(&o[F::out_elem(k, d)], x);
+                    else o[F::out_elem(k, d)] = x;
+                });
+            }
+        } else {
+            F::template passes<0, true, false>(in, out, tw, lds, ibase, obase, d, l0, false);
+            __syncthreads();
+            const T half = (T)0.5;
+            auto untangle = [&](int line, int k) {
+                const cx<T> a = lds[line * F::LD + F::lidx(k == M ? 0 : k)];
+                const cx<T> b = conj(lds[line * F::LD + F::lidx(k == 0 ? 0 : M - k)]);
+                const cx<T> s = a + b, df = a - b;
+                const cx<T> w = twmul(df, rtw[k]);                            // W^k (Z_k - conj Z_{M-k})
+                const cx<T> x = mk(half * (s.x + w.y), half * (s.y - w.x));  // (s - i w) / 2
+                // non-temporal (measured on MI355X, 1024 x 512 x 256 FP64 R2C rows: 394 against
+                // 399-403 us; FP32 unchanged within the noise)
+                store_nt(&out[obase + (i64)line * d.out_ls + F::out_elem(k, d)], x);
+            };
+            // LPB * M items, fully unrolled; the thread of k = 0 also writes X_M, so the loop has
+            // no mostly idle last round (measured on MI355X, 1024 x 512 x 256: FP32 rows 239
+            // against 254 us, FP64 380 against 397 us for a loop over LPB * (M + 1) items)
+            constexpr int UIT = (LPB * M + F::NT - 1) / F::NT;
+#pragma unroll
+            for (int q = 0; q < UIT; q++) {
+                const int e = (int)threadIdx.x + q * F::NT;
+                if (UIT * F::NT == LPB * M || e < LPB * M) {
+                    const int line = e / M, k = e % M;
+                    if (l0 + line < d.nl) {
+                        untangle(line, k);
+                        if (k == 0) untangle(line, M);
+                    }
                 }
             }
         }
@@ -785,43 +909,71 @@ fft_r2c_kernel(const cx<T>* __restrict__ in, cx<T>* __restrict__ out,
 // stride in_ns) -- the transpose that precedes the C2R pass is fused into its load.
 // TWL: persistent blocks copy both twiddle tables into LDS once (as fft_c2c_kernel's TWL).
 namespace dtfft {
-template <typename T, class S, int TPL, int LPB, int PAD, bool IN_COLS>
+template <typename T, class S, int TPL, int LPB, int PAD, bool IN_COLS, bool TWL>
 struct c2r_tiles {
     typedef fft_tile<T, S, TPL, LPB, false, false, PAD> F;
     typedef typename tw_of<T>::type tw_t;
     static __device__ __forceinline__ void run(const cx<T>* __restrict__ in, cx<T>* __restrict__ out,
-                                               const tw_t* tw, const tw_t* rtw, cx<T>* lds, const lines_desc& d) {
+                                               const tw_t* tw_, const tw_t* rtw_, cx<T>* lds, const lines_desc& d) {
     constexpr int M = S::N;
     for (i64 t = blockIdx.x; t < d.ntiles; t += gridDim.x) {
         i64 l0, ibase, obase;
         F::tile_bases(d, t, l0, ibase, obase);
-        for (int e = threadIdx.x; e < LPB * M; e += F::NT) {
-            int line, k;
-            if constexpr (IN_COLS) { line = e % LPB; k = e / LPB; }
-            else { line = e / M; k = e % M; }
-            cx<T> z = mk((T)0, (T)0);
-            if (l0 + line < d.nl) {
-                const i64 lb = ibase + (i64)line * d.in_ls;
-                cx<T> a, b;
-                if constexpr (IN_COLS) {
-                    a = in[lb + (i64)k * d.in_ns];
-                    b = in[lb + (i64)(M - k) * d.in_ns];
-                } else {
-                    a = in[lb + k];
-                    b = in[lb + (M - k)];
+        const tw_t *tw = tw_, *rtw = rtw_;
+        if constexpr (!TWL) { tw = fresh(tw); rtw = fresh(rtw); }
+        if constexpr (F::NP > 1 && S::radix(0) <= 16) {
+            // the folding on mirror pairs in the registers of the first pass
+            constexpr int R = S::radix(0);
+            typedef mirror_pairs<T, S, R> P;
+            const int line = IN_COLS ? threadIdx.x % LPB : threadIdx.x / TPL;
+            const int j = IN_COLS ? threadIdx.x / LPB : threadIdx.x % TPL;
+            const bool live = l0 + line < d.nl;
+            const cx<T>* x = in + ibase + (i64)line * d.in_ls;
+            const i64 es = IN_COLS ? d.in_ns : 1;
+#pragma unroll 1
+            for (int u = j; u < P::UNITS; u += TPL) {
+                cx<T> v[2][R];
+                P::fold(u, v[0], v[1], rtw, [&](int k) { return live ? x[(i64)k * es] : mk((T)0, (T)0); });
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    bfly<T, R>::run(v[q]);
+                    const int b = q ? P::second(u) : u;
+                    if (q == 0 || P::EVEN || u != 0) {
+#pragma unroll
+                        for (int s = 0; s < R; s++) lds[line * F::LD + F::lidx(b * R + s)] = v[q][s];
+                    }
                 }
-                if (k == 0) { a.y = (T)0; b.y = (T)0; }  // Im X_0, Im X_M do not contribute
-                b = conj(b);
-                const cx<T> e2 = a + b;
-                const cx<T> o2 = twmul(a - b, conj_tw(rtw[k]));
-                z = mk(e2.x - o2.y, e2.y + o2.x);  // 2E + i 2O
             }
-            // backward transform = conj(forward(conj z)): store conj(z); the last pass
-            // conjugates on its global write (inv = true)
-            lds[line * F::LD + F::lidx(k)] = conj(z);
+            F::template passes<1, false, true>(in, out, tw, lds, ibase, obase, d, l0, true);
+        } else {
+            for (int e = threadIdx.x; e < LPB * M; e += F::NT) {
+                int line, k;
+                if constexpr (IN_COLS) { line = e % LPB; k = e / LPB; }
+                else { line = e / M; k = e % M; }
+                cx<T> z = mk((T)0, (T)0);
+                if (l0 + line < d.nl) {
+                    const i64 lb = ibase + (i64)line * d.in_ls;
+                    cx<T> a, b;
+                    if constexpr (IN_COLS) {
+                        a = in[lb + (i64)k * d.in_ns];
+                        b = in[lb + (i64)(M - k) * d.in_ns];
+                    } else {
+                        a = in[lb + k];
+                        b = in[lb + (M - k)];
+                    }
+                    if (k == 0) { a.y = (T)0; b.y = (T)0; }  // Im X_0, Im X_M do not contribute
+                    b = conj(b);
+                    const cx<T> e2 = a + b;
+                    const cx<T> o2 = twmul(a - b, conj_tw(rtw[k]));
+                    z = mk(e2.x - o2.y, e2.y + o2.x);  // 2E + i 2O
+                }
+                // backward transform = conj(forward(conj z)): store conj(z); the last pass
+                // conjugates on its global write (inv = true)
+                lds[line * F::LD + F::lidx(k)] = conj(z);
+            }
+            __syncthreads();
+            F::template passes<0, false, true>(in, out, tw, lds, ibase, obase, d, l0, true);
         }
-        __syncthreads();
-        F::template passes<0, false, true>(in, out, tw, lds, ibase, obase, d, l0, true);
         __syncthreads();
     }
     }
@@ -833,7 +985,7 @@ __global__ void __launch_bounds__(TPL * LPB)
 fft_c2r_kernel(const cx<T>* __restrict__ in, cx<T>* __restrict__ out,
                const typename tw_of<T>::type* __restrict__ tw,
                const typename tw_of<T>::type* __restrict__ rtw, dtfft::lines_desc d) {
-    typedef dtfft::c2r_tiles<T, S, TPL, LPB, PAD, IN_COLS> K;
+    typedef dtfft::c2r_tiles<T, S, TPL, LPB, PAD, IN_COLS, TWL> K;
     typedef typename tw_of<T>::type tw_t;
     __shared__ cx<T> lds[K::F::LDS_ELEMS];
     if constexpr (TWL) {

@@ -11,6 +11,7 @@
 // padding come from a heuristic or, at effort >= MEASURE, from timing the candidates
 // on the device (the project's replacement for dtfft_nvrtc_block_optimizer).
 #include <algorithm>
+#include <numeric>
 #include <array>
 #include <cmath>
 #include <functional>
@@ -266,10 +267,9 @@ void apply_twl(fft_config& c, const lines_desc& d, int mode) {
         // At n = 512 the one-tile-per-block launch stays faster (384 against 412 us).  FP32
         // column-in passes without LDS-DMA (e.g. 513 lines per row, the complex X pencil of an
         // R2C plan) run one 1024-thread block per CU anyway, so persistence costs no occupancy:
-        // 1024 x 512 x 256 R2C's X->Y pass went from 325 to 276 us; the fused Z->X C2R of the
-        // same plan from 453 to 386 us.  FP64 measured no gain.
+        // 1024 x 512 x 256 R2C's X->Y pass went from 325 to 276 us.  FP64 measured no gain.
         const bool rows = c.kind == 0 && !c.in_cols && !c.out_cols;
-        const bool cols = (c.kind == 0 && c.in_cols && c.seg == 0) || (c.kind == 2 && c.in_cols);
+        const bool cols = c.kind == 0 && c.in_cols && c.seg == 0;
         want = !c.dbl && ntiles >= 2048 && ((rows && c.n >= 2048) || cols);
     }
     if (!want) return;
@@ -917,6 +917,42 @@ int32_t plan_fft_stage(int n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, i
     return st->init(cfg, d);
 }
 
+// Schedule and threads per line of the half-length transform (m points) of a real line, R2C order.
+// The last pass runs on mirror pairs, two butterflies a thread, so its radix sets the threads: 4
+// gives 8 points to each, where 16 points leave too few waves (registers) and 4 too many passes
+// (rows, us per GiB, FP32 / FP64: 512 points 8 4 4 4 on 64 threads 200 / 176, 8 8 8 on 32 threads
+// 222 / 183, on 64 threads 281 / 218; 128 points 8 4 4 203 / 179, 16 8 247 / 202).  Lines under 64
+// points take 2 or 3 (32 points: 4 4 2 222 / 178, 8 4 261 / 205).  The other passes: the fewest of
+// radices up to 10, as equal as they come.  False: m in one pass.
+static bool real_schedule(int m, bool dbl, std::vector<int>& radices, int& tpl) {
+    if (!factorize(m, radices) || radices.size() < 2) return false;
+    int last = 0;
+    for (int r : m < 64 ? std::vector<int>{3, 2, 5, 7, 11, 13} : std::vector<int>{4, 3, 5, 2, 7, 11, 13})
+        if (!last && m % r == 0) last = r;
+    std::vector<int> cur, best;
+    std::function<void(int, int)> rec = [&](int k, int hi) {
+        if (k == 1) {
+            const int a = std::accumulate(cur.begin(), cur.end(), 0), b = std::accumulate(best.begin(), best.end(), 0);
+            if (best.empty() || cur.size() < best.size() || (cur.size() == best.size() && a < b)) best = cur;
+            return;
+        }
+        if (cur.size() >= 8 || (!best.empty() && cur.size() >= best.size())) return;
+        for (int r = std::min(hi, 13); r >= 2; r--)
+            if (k % r == 0 && (r <= 10 || r == 11 || r == 13)) {
+                cur.push_back(r);
+                rec(k / r, r);
+                cur.pop_back();
+            }
+    };
+    rec(m / last, 13);
+    if (best.empty()) return false;
+    radices = best;
+    radices.push_back(last);
+    tpl = (m / last + 1) / 2;
+    if (tpl > (dbl ? 128 : 64)) tpl = (tpl + 1) / 2;
+    return true;
+}
+
 int32_t plan_real_stage(int kind, int n, bool dbl, int64_t how_many, int64_t idist, int64_t odist, int effort,
                         hipStream_t stream, fft_stage* st) {
     (void)effort; (void)stream;
@@ -944,12 +980,17 @@ int32_t plan_real_stage(int kind, int n, bool dbl, int64_t how_many, int64_t idi
     c.kind = kind;
     if (m == 1) {
         c.radices = {1}; c.tpl = 1; c.lpb = 64;
+    } else if (real_schedule(m, dbl, rad, c.tpl)) {
+        c.radices = rad;
+        if (kind == 2) std::reverse(c.radices.begin(), c.radices.end());
+        // about two waves per block, as full as they come
+        auto full = [&](int l) { return (double)(l * c.tpl) / (double)((l * c.tpl + 63) / 64 * 64); };
+        c.lpb = std::max(1, 128 / c.tpl);
+        for (int l = c.lpb + 1; l * c.tpl <= 256; l++)
+            if (full(l) > full(c.lpb) + 0.04) c.lpb = l;
     } else if (factorize(m, rad)) {
-        // one butterfly per thread and pass: the untangling adds registers to the row FFT, and
-        // fewer per thread keep more waves resident
         pick_schedule(m, 8, c.radices, c.tpl);
         c.lpb = std::max(1, (c.tpl >= 64 ? 256 : 128) / c.tpl);
-        while (c.tpl > 1024) c.tpl = (c.tpl + 1) / 2;
     }
     lines_desc d;
     if (kind == 1) {  // real lines (idist reals) viewed as complex; complex out (odist)
@@ -983,17 +1024,20 @@ int32_t plan_c2r_cols_stage(int n, bool dbl, int64_t nl, int64_t nb, int64_t in_
     }
     c = default_fft_config(m, dbl, true, false, nl * nb, nl);
     c.kind = 2;
+    const fft_config whole = c;  // the schedule of the LDS-DMA kernels
+    if (real_schedule(m, dbl, rad, c.tpl)) {
+        c.radices.assign(rad.rbegin(), rad.rend());
+        while (c.tpl * c.lpb > 1024 && c.lpb > 1) c.lpb /= 2;
+    }
     lines_desc d = make_lines(nl, nb, 1, in_bs, in_ns, out_ls, out_bs, 1, c.lpb);
-    // persistent blocks with both twiddle tables in LDS by the configuration's rule (FP32 by
-    // default: one 1024-thread block per CU either way)
-    apply_twl(c, d, global_config().twl);
+    apply_twl(c, d, global_config().twl);  // the tables in LDS only when forced (no gain measured)
     if (lds_dma != 0) {
         // LDS-DMA kernels: 128-byte input row pieces loaded straight into LDS, each read once;
         // two butterflies per thread and pass.  lds_dma 2: the persistent double buffer
         // (fft_c2r_dma2_kernel, one block per CU); 3: one tile per block (fft_c2r_dma_kernel,
         // two blocks per CU, the FFT twiddles in LDS only when forced with twl = 2, which leaves
         // room for one block per CU); 1: the double buffer where it fits, else one tile per block
-        fft_config x = c;
+        fft_config x = whole;
         x.lpb = 128 / elem_bytes(dbl);
         x.pad = 1;
         const int rmax = *std::max_element(x.radices.begin(), x.radices.end());
