@@ -261,16 +261,18 @@ void apply_twl(fft_config& c, const lines_desc& d, int mode) {
     const int64_t ntiles = ((d.nl + c.lpb - 1) / c.lpb) * d.nb;
     bool want = mode >= 2;
     if (mode == 1) {
-        // Default rule, measured on MI355X.  Long FP32 rows (n >= 2048, plain or fused
+        // Default rule, measured on MI355X.  Long FP32 rows (n > 1024, plain or fused
         // unpack+FFT): the table (n - 1 entries of 16 bytes) otherwise shares the L1 cache with
-        // the tile; the 2048-point rows of a 2048 x 512 x 512 pencil went from 2028 to 1702 us.
-        // At n = 512 the one-tile-per-block launch stays faster (384 against 412 us).  FP32
+        // the tile; the 2048-point rows of a 2048 x 512 x 512 pencil went from 2028 to 1702 us,
+        // 1280-point rows from 445 to 375 us per 2 GiB.  At n = 512 and 1024 the one-tile-per-block
+        // launch stays faster (384 against 412 us, 360 against 367), and at 4096, where the table
+        // leaves room for one block per CU (460 against 504 us).  FP32
         // column-in passes without LDS-DMA (e.g. 513 lines per row, the complex X pencil of an
         // R2C plan) run one 1024-thread block per CU anyway, so persistence costs no occupancy:
         // 1024 x 512 x 256 R2C's X->Y pass went from 325 to 276 us.  FP64 measured no gain.
         const bool rows = c.kind == 0 && !c.in_cols && !c.out_cols;
         const bool cols = c.kind == 0 && c.in_cols && c.seg == 0;
-        want = !c.dbl && ntiles >= 2048 && ((rows && c.n >= 2048) || cols);
+        want = !c.dbl && ntiles >= 2048 && ((rows && c.n > 1024 && c.n != 4096) || cols);
     }
     if (!want) return;
     c.twl = 1;
@@ -321,6 +323,25 @@ void pick_schedule(int n, int points, std::vector<int>& radices, int& tpl) {
     known[{n, tpl}] = radices;
 }
 
+// n as four radices up to 10, as equal as they come: the passes of long rows.  Three of up to 16
+// hold more registers per thread than leave enough waves (rows, us per 2 GiB, three / four passes:
+// 1280 points FP32 509 / 375, FP64 449 / 348; 2048 points FP64 369 / 343; 3072 points FP64 402 / 375;
+// 4096 points FP32 557 / 460).  2048 points FP32 stay with 16 16 8 on 128 threads (381 / 373, but
+// the unpacking of a 2048 x 512 x 512 pencil 1685 / 1735).
+static bool four_passes(int n, std::vector<int>& radices) {
+    int sum = 1 << 30;
+    for (int a = 10; a >= 2; a--)
+        for (int b = a; b >= 2; b--)
+            for (int e = b; e >= 2; e--) {
+                if (n % (a * b * e) != 0) continue;
+                const int f = n / (a * b * e);
+                if (f < 2 || f > e || a + b + e + f >= sum) continue;
+                sum = a + b + e + f;
+                radices = {a, b, e, f};
+            }
+    return sum < 1 << 30;
+}
+
 fft_config default_fft_config(int n, bool dbl, bool in_cols, bool out_cols, int64_t lines, int64_t nl) {
     fft_config c;
     c.n = n; c.dbl = dbl; c.in_cols = in_cols; c.out_cols = out_cols;
@@ -364,6 +385,10 @@ fft_config default_fft_config(int n, bool dbl, bool in_cols, bool out_cols, int6
         // 256 MB; FP64 79 and 84 us)
         c.pad = 0;
         c.lpb = std::max(1, (c.tpl >= 128 ? 256 : 128) / c.tpl);
+        if (!few && n >= 1024 && n <= 4096 && (dbl || n != 2048) && four_passes(n, c.radices)) {
+            c.tpl = n == 1024 && !dbl ? 64 : n <= 2048 ? 128 : 256;
+            c.lpb = !dbl && n > 2048 && n <= 2560 ? 2 : 1;
+        }
         if (few) while (c.lpb > 1 && c.tpl * c.lpb >= 128 && lines / c.lpb < 512) c.lpb /= 2;
     }
     while (c.tpl * c.lpb > 1024 && c.lpb > 1) c.lpb /= 2;
