@@ -7,7 +7,8 @@
 //   backward: FFT_Z (in -> aux), Z->X + FFT_X (aux -> out), FFT_Y in place (out)
 // Within a stage the grids are grouped by the length of the stage's axis.  Each group is
 // one persistent launch of a kernel compiled for that length alone (so its register budget
-// is that of a single-length kernel), walking a work list of (grid, tile) items.  The groups
+// is that of a single-length kernel), walking a work list of (grid, tile) items; FP32 column
+// groups load their tiles straight into LDS where the grids' rows allow it.  The groups
 // of a stage are independent: they are spread over side streams, forked from and joined
 // back to the caller's stream with events, so that small groups overlap.  The
 // forward+backward cycle is captured once as a hipGraph (the forks become parallel

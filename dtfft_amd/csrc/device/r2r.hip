@@ -26,10 +26,11 @@
 // them is t4(j) = e^{-i pi j / 4n} or its conjugate, j < 2n; the fused kernel reads them from
 // a table of that function, the three-launch path evaluates it in place.
 //
-// Lines of unit element stride take the fused kernel fft_r2r_kernel: the real lines go to
-// LDS, the pre-process fills the complex work line in LDS, the Stockham passes of fft_tile
-// run there, and the post-process writes the real outputs: one read and one write of each
-// real element.  Other strides take the three launches through a complex work buffer.
+// Powers of two of types 2 and 3 take the persistent fft_r2r_kernel: the real lines go to LDS, the
+// pre-process fills the complex work line in LDS, the Stockham passes of fft_tile run there, and
+// the post-process writes the real outputs.  Every other length whose work length has radices takes
+// r2r_tile_kernel, with any strides.  Both read and write each real element once.  The rest
+// (a prime without a radix in the work length) takes the three launches through a complex buffer.
 #include "fft.hip"  // fft_tile: the Stockham passes, here run on work lines held in LDS
 
 struct r2r_desc {
