@@ -190,9 +190,10 @@ struct r2r_desc_h {
     int64_t out_seg;  // chunk-blocked row output: chunk stride (kernel built with OSEG)
 };
 // One R2R transform (DCT/DST 1-4, FFTW kinds 3..10) over nl x nb real lines of length n:
-// pre-process -> complex FFT of length m -> post-process.  Lines of unit element stride
-// with the same layout in and out take one fused launch (fft_r2r_kernel); otherwise three
-// launches through a caller-owned work buffer of work_bytes().
+// pre-process -> complex FFT of length m -> post-process, in one launch (fft_r2r_kernel,
+// r2r_tile_kernel) or in three through a caller-owned work buffer of work_bytes().  A stage whose
+// lines are spaced differently in and out holds both: the one launch for buffers apart, the three
+// for buffers that overlap (in place).
 struct r2r_stage {
     int kind = 0;
     int64_t n = 0, m = 0;
@@ -212,6 +213,8 @@ struct r2r_stage {
     unsigned fgrid = 0, fblock = 0;
     int32_t init(int kind, int64_t n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, int64_t in_bs,
                  int64_t in_es, int64_t out_ls, int64_t out_bs, int64_t out_es, int effort, hipStream_t stream);
+    int32_t init_launches(int effort, hipStream_t stream);
+    bool overlap(const void* in, const void* out) const;
     // The fused kernel reading its lines across (nl adjacent lines per batch, element stride
     // in_es) and writing rows (out_es 1) or, with out_cols, columns (out_ls 1) -- the transpose
     // before the stage fused into its load.  Types 2 / 3 of even length through the half-length

@@ -4,8 +4,9 @@
 // is r2r_pre (real line -> complex line of length M), the Stockham C2C transform of the
 // work line, and r2r_post (complex -> n real outputs); device/r2r.hip lists the per-kind
 // maps.  One kernel runs all three through LDS (init, init_cols: persistent, types 2 and 3 of even
-// length; init_tile: every kind and layout); work lengths without a schedule run three launches
-// through a work buffer (lines x M complex) that belongs to the caller.
+// length; init_tile: every kind and layout); work lengths without a schedule, and lines spaced
+// differently in and out whose buffers overlap, run three launches through a work buffer (lines x M
+// complex) that belongs to the caller.
 #include <map>
 #include <mutex>
 
@@ -98,13 +99,15 @@ int32_t r2r_stage::init(int kind_, int64_t n_, bool dbl_, int64_t nl, int64_t nb
     const bool half_ok = (kind == 4 || kind == 5 || kind == 8 || kind == 9) && n % 2 == 0 && n >= 8 &&
                          half_schedule((int)(n / 2), hrad);
     const int64_t mf = n / 2;  // length of its FFT
+    // spaced alike in and out: in place, a block overwrites the lines that it has read itself
+    const bool same = in_ls == out_ls && in_bs == out_bs && in_es == out_es;
     bool ok = false;
     if ((n & (n - 1)) != 0) {
         // the persistent kernel below, with its radix-4 passes, is the faster form for powers of
         // two only (512 MB FP32 DCT-2 / DCT-3 rows: 128 points 253 / 209 us against 280 / 228;
         // 384 points 422 / 395 us against 333 / 285)
         TRY(init_tile(kind, n, dbl, nl, nb, in_ls, in_bs, in_es, out_ls, out_bs, out_es, &ok));
-        if (ok) return DTFFT_HIP_SUCCESS;
+        if (ok) return same ? DTFFT_HIP_SUCCESS : init_launches(effort, stream);
     }
     if (half_ok && in_es == 1 && out_es == 1 && in_ls == out_ls && in_bs == out_bs && even) {
         fft_config c = default_fft_config((int)mf, dbl, false, false, nl * nb, nl);
@@ -150,13 +153,17 @@ int32_t r2r_stage::init(int kind_, int64_t n_, bool dbl_, int64_t nl, int64_t nb
         }
     }
     TRY(init_tile(kind, n, dbl, nl, nb, in_ls, in_bs, in_es, out_ls, out_bs, out_es, &ok));
-    if (ok) return DTFFT_HIP_SUCCESS;
-    // A work length with a prime that no radix covers (or one that does not fit) runs three
-    // launches, whose C2C stage is the Bluestein form of plan_fft_stage.
-    const std::string h = half ? ", true>" : ", false>";
+    if (ok && same) return DTFFT_HIP_SUCCESS;
+    return init_launches(effort, stream);
+}
+
+// The three launches over the lines of d: where there is no kernel that runs all of it, and beside
+// r2r_tile_kernel where the lines are spaced differently in and out.
+int32_t r2r_stage::init_launches(int effort, hipStream_t stream) {
+    const std::string t = dbl ? "double" : "float", h = half ? ", true>" : ", false>";
     TRY(rtc_get("r2r", "r2r_pre<" + t + ", " + std::to_string(kind) + h, &pre));
     TRY(rtc_get("r2r", "r2r_post<" + t + ", " + std::to_string(kind) + h, &post));
-    return plan_fft_stage((int)m, dbl, nl * nb, 1, m, 0, 1, m, 0, 1, true, effort, stream, &fft);
+    return plan_fft_stage((int)m, dbl, d.nl * d.nb, 1, m, 0, 1, m, 0, 1, true, effort, stream, &fft);
 }
 
 int32_t r2r_stage::init_tile(int kind_, int64_t n_, bool dbl_, int64_t nl, int64_t nb, int64_t in_ls, int64_t in_bs,
@@ -259,7 +266,7 @@ int32_t r2r_stage::blocked_pair(const r2r_stage& rows, const r2r_stage& cols, r2
     return DTFFT_HIP_SUCCESS;
 }
 
-size_t r2r_stage::work_bytes() const { return fused ? 0 : (size_t)(d.nl * d.nb * d.wdist) * (dbl ? 16 : 8); }
+size_t r2r_stage::work_bytes() const { return pre ? (size_t)(d.nl * d.nb * d.wdist) * (dbl ? 16 : 8) : 0; }
 
 int32_t r2r_stage::init_cols(int kind_, int64_t n_, bool dbl_, int64_t nl, int64_t nb, int64_t in_bs, int64_t in_es,
                              int64_t out_ls, int64_t out_bs, int64_t out_es, bool out_cols, bool* ok) {
@@ -346,9 +353,19 @@ static unsigned grid_for(int64_t items) {
     return (unsigned)std::max<int64_t>(1, std::min<int64_t>((items + 255) / 256, 1 << 20));
 }
 
+// Whether the lines read and the lines written share memory, taken from the first to the last.
+bool r2r_stage::overlap(const void* in, const void* out) const {
+    auto end = [&](const void* p, int64_t ls, int64_t bs, int64_t es) {
+        return (uintptr_t)p + (uintptr_t)((d.nl - 1) * ls + (d.nb - 1) * bs + (n - 1) * es + 1) * (dbl ? 8 : 4);
+    };
+    return (uintptr_t)in < end(out, d.out_ls, d.out_bs, d.out_es) && (uintptr_t)out < end(in, d.in_ls, d.in_bs, d.in_es);
+}
+
 int32_t r2r_stage::run(const void* in, void* out, void* work, hipStream_t s) const {
     if (d.nl * d.nb == 0) return DTFFT_HIP_SUCCESS;
-    if (fused) {
+    // Where both forms are set up the lines move: a block of the one launch would write lines that
+    // other blocks have yet to read.
+    if (fused && !(pre && overlap(in, out))) {
         r2r_desc_h dd = d;
         void* twp = ftw ? ftw->ptr : nullptr;
         void* tp = t4 ? t4->ptr : nullptr;
