@@ -591,6 +591,7 @@ struct line_passes {
     static __device__ __forceinline__ void run(const tw_t* __restrict__ tw, const Load& load, const Store& store) {
         constexpr int R = S::radix(p), L = S::span(p), TWO = S::tw_off(p);
         constexpr int NB = S::N / R, IT = (NB + TPL - 1) / TPL;
+        static_assert(R <= 16 || sizeof(T) == 4, "FP64 keeps to radices up to 16 here (r2r.cpp, init_tile)");
         int line, j;
         map<COLS>(line, j);
         cx<T> v[IT][R];

@@ -177,7 +177,9 @@ int32_t r2r_stage::init_tile(int kind_, int64_t n_, bool dbl_, int64_t nl, int64
     c.n = (int)M;
     c.dbl = dbl_;
     c.pad = 1;
-    if (large_schedule((int)M, dbl_, kMaxPrime(dbl_), c.radices))
+    // A prime above 13 in FP64 is left to the three launches: line_passes with a radix-31 butterfly in
+    // FP64 has faulted a card (in another kernel), and the cause is not known.
+    if (!dbl_ && large_schedule((int)M, false, kMaxPrime(false), c.radices))
         c.tpl = (int)std::max(M / c.radices[0], (M + 23) / 24);
     else if (factorize((int)M, c.radices))
         pick_schedule((int)M, 8, c.radices, c.tpl);
