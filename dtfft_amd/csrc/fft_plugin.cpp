@@ -978,6 +978,7 @@ static bool real_schedule(int m, bool dbl, std::vector<int>& radices, int& tpl) 
     radices.push_back(last);
     tpl = (m / last + 1) / 2;
     if (tpl > (dbl ? 128 : 64)) tpl = (tpl + 1) / 2;
+    while (tpl > 1024) tpl = (tpl + 1) / 2;  // a block's most threads
     return true;
 }
 
