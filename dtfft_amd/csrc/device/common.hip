@@ -57,6 +57,18 @@ __device__ __forceinline__ cx<double> twmul(cx<double> a, const cx<double> w) {
     return mk(re, im);
 }
 
+// c + i s as a twiddle, from FP64 values known at compile time
+template <typename T> __device__ __forceinline__ typename tw_of<T>::type tw_const(double c, double s) {
+    if constexpr (sizeof(T) == 8) {
+        return mk(c, s);
+    } else {
+        twf w;
+        w.rh = (float)c; w.rl = (float)(c - (double)w.rh);
+        w.ih = (float)s; w.il = (float)(s - (double)w.ih);
+        return w;
+    }
+}
+
 // Non-temporal store of one complex value (streaming output that no later instruction of the
 // kernel reads back).  Measured on MI355X at 512^3 FP32: the LDS-DMA column-in / row-out pass
 // went from 430 to 422 us with its row stores non-temporal, the row passes from 377-395 to
