@@ -254,6 +254,9 @@ static bool valid(const fft_config& c) {
     return true;
 }
 
+// Whether two blocks of the kernel fit the LDS of a CU.
+static bool two_blocks(const fft_config& c) { return 2 * fft_lds_bytes(c) <= kMaxLds; }
+
 void apply_twl(fft_config& c, const lines_desc& d, int mode) {
     c.twl = 0;
     // the LDS-DMA column kernels keep their twiddles in LDS anyway; R2C rows have no such form
@@ -263,16 +266,18 @@ void apply_twl(fft_config& c, const lines_desc& d, int mode) {
     if (mode == 1) {
         // Default rule, measured on MI355X.  Long FP32 rows (n > 1024, plain or fused
         // unpack+FFT): the table (n - 1 entries of 16 bytes) otherwise shares the L1 cache with
-        // the tile; the 2048-point rows of a 2048 x 512 x 512 pencil went from 2028 to 1702 us,
-        // 1280-point rows from 445 to 375 us per 2 GiB.  At n = 512 and 1024 the one-tile-per-block
-        // launch stays faster (384 against 412 us, 360 against 367), and at 4096, where the table
-        // leaves room for one block per CU (460 against 504 us).  FP32
+        // the tile (us per 2 GiB, global / LDS table: 1280 points 508 / 441, 2048 points 468 / 406,
+        // 3200 points 567 / 490).  At n = 512 and 1024 the one-tile-per-block launch stays faster
+        // (384 against 412 us, 398 against 528), and where tile and table leave room for one block
+        // per CU only (3600 points 573 / 745, 4096 points 522 / 722).  FP32
         // column-in passes without LDS-DMA (e.g. 513 lines per row, the complex X pencil of an
         // R2C plan) run one 1024-thread block per CU anyway, so persistence costs no occupancy:
         // 1024 x 512 x 256 R2C's X->Y pass went from 325 to 276 us.  FP64 measured no gain.
         const bool rows = c.kind == 0 && !c.in_cols && !c.out_cols;
         const bool cols = c.kind == 0 && c.in_cols && c.seg == 0;
-        want = !c.dbl && ntiles >= 2048 && ((rows && c.n > 1024 && c.n != 4096) || cols);
+        fft_config t = c;
+        t.twl = 1;
+        want = !c.dbl && ntiles >= 2048 && ((rows && c.n > 1024 && two_blocks(t)) || cols);
     }
     if (!want) return;
     c.twl = 1;
@@ -323,11 +328,10 @@ void pick_schedule(int n, int points, std::vector<int>& radices, int& tpl) {
     known[{n, tpl}] = radices;
 }
 
-// n as four radices up to 10, as equal as they come: the passes of long rows.  Three of up to 16
-// hold more registers per thread than leave enough waves (rows, us per 2 GiB, three / four passes:
-// 1280 points FP32 509 / 375, FP64 449 / 348; 2048 points FP64 369 / 343; 3072 points FP64 402 / 375;
-// 4096 points FP32 557 / 460).  2048 points FP32 stay with 16 16 8 on 128 threads (381 / 373, but
-// the unpacking of a 2048 x 512 x 512 pencil 1685 / 1735).
+// n as four radices up to 10, as equal as they come: the passes of long rows whose three passes of up
+// to 16 hold more registers per thread than leave enough waves (rows, us per 2 GiB, three / four passes:
+// 1280 points FP32 513 / 441, FP64 452 / 396; 1536 points FP32 469 / 447, FP64 424 / 378; 2560 points
+// FP32 534 / 467; 4096 points FP32 588 / 522, FP64 416 / 399).
 static bool four_passes(int n, std::vector<int>& radices) {
     int sum = 1 << 30;
     for (int a = 10; a >= 2; a--)
@@ -385,9 +389,21 @@ fft_config default_fft_config(int n, bool dbl, bool in_cols, bool out_cols, int6
         // 256 MB; FP64 79 and 84 us)
         c.pad = 0;
         c.lpb = std::max(1, (c.tpl >= 128 ? 256 : 128) / c.tpl);
-        if (!few && n >= 1024 && n <= 4096 && (dbl || n != 2048) && four_passes(n, c.radices)) {
-            c.tpl = n == 1024 && !dbl ? 64 : n <= 2048 ? 128 : 256;
-            c.lpb = !dbl && n > 2048 && n <= 2560 ? 2 : 1;
+        std::vector<int> four;
+        if (!few && n >= 1024 && n <= 4096 && four_passes(n, four)) {
+            const int tpl = n <= 2048 ? 128 : 256;
+            // FP32: where the schedule above holds up to 16 points a thread it is the faster one (us per
+            // 2 GiB, that / four radices up to 10: 1792 points 420 / 552, 1920 points 419 / 540, 2048
+            // points 406 / 465, 3200 points 490 / 549, 3360 points 432 / 522), unless the twiddles are not
+            // in LDS and the four leave no more threads idle (4096 points 588 / 522, 3600 points 573 / 705)
+            fft_config t = c;
+            t.twl = 1;
+            const bool few_points = !dbl && n <= 16 * c.tpl;
+            if (!few_points || (!two_blocks(t) && idle_factor(four, n, tpl) <= idle_factor(c.radices, n, c.tpl))) {
+                c.radices = four;
+                c.tpl = tpl;
+                c.lpb = !dbl && n > 2048 && n <= 2560 ? 2 : 1;
+            }
         }
         if (few) while (c.lpb > 1 && c.tpl * c.lpb >= 128 && lines / c.lpb < 512) c.lpb /= 2;
     }
