@@ -482,7 +482,7 @@ std::vector<fft_config> fft_candidates(int n, bool dbl, bool in_cols, bool out_c
     // threads per line of its own largest radix (one and two butterflies per thread and pass)
     // and the default's lines per block and padding
     const auto scheds = radix_schedules(n, 4);
-    for (size_t i = 1; i < scheds.size(); i++) {
+    for (size_t i = 0; i < scheds.size(); i++) {
         const int rmax = *std::max_element(scheds[i].begin(), scheds[i].end());
         for (int t : {n / rmax, n / rmax / 2}) {
             if (t < 1) continue;
@@ -826,6 +826,41 @@ fft_config dma_config(const fft_config& cfg, int dma) {
     return c;
 }
 
+// Takes a column-in stage from its plain configuration to the LDS-DMA one where it is forced (lds_dma 2
+// or 3) or the default rule has it so, or to the wide plain form; false: cfg stays.
+static bool cols_config(fft_config& cfg, const lines_desc& d, bool inplace, int lds_dma) {
+    if (lds_dma == 0 || (lds_dma == 1 && cfg.dbl)) return false;
+    // Default for FP32 column-in passes, us per 2 GiB, LDS-DMA (one tile per block) against the
+    // plain column kernel: 16 points 354 / 404, 36 points 384 / 550, 64 points 346 / 395, 210
+    // points 380 / 490, 320 points 374 / 500, 512 points 384 / 442, 900 points 536 / 662; rows
+    // of 210 lines, whose pieces straddle 128-byte lines: 64 points 357 / 441, 320 points 419 /
+    // 514, 512 points 461 / 536.  In place from 48 points on (60 points 394 / 453, 36 points 467 /
+    // 408, 512 points 395 / 453).  Launches of few tiles are bound by latency, where the plain
+    // kernel's loads go straight to the first pass (256 points, 4 MB: 5.9 / 5.2).  FP64 keeps
+    // the plain kernel, which the autotuner preferred there.
+    const fft_config c = dma_config(cfg, lds_dma == 2 ? 1 : 2);
+    const bool use = lds_dma >= 2 || (d.nl * d.nb >= 8192 && cfg.n >= (c.out_cols ? 48 : 16));
+    if (lds_dma == 1 && inplace && cfg.out_cols && cfg.n >= 512) {
+        // In-place FP32 column passes of n >= 512 where a 32-line tile (256-byte pieces of
+        // every row) fits with the LDS twiddle table: the plain kernel, persistent, four
+        // butterflies per thread and pass.  EXHAUSTIVE picked it at 512^3 in three runs,
+        // 416 us against 427 us for the LDS-DMA double buffer (the 32-line tile fits only
+        // up to n = 512; at 256^3 and 384^3 the tuner picked other kernels, which keep the
+        // rule below).
+        fft_config w = cfg;
+        const int rmax = *std::max_element(w.radices.begin(), w.radices.end());
+        w.dma = 0;
+        w.lpb = 32;
+        w.pad = 1;
+        w.tpl = std::max(1, cfg.n / rmax / 4);
+        apply_twl(w, d, 1);  // the measured form: persistent with LDS twiddles (>= 2048 tiles)
+        if (w.twl && valid(w)) { cfg = w; return true; }
+    }
+    if (!use || !dma_ok(c, d)) return false;
+    cfg = c;
+    return true;
+}
+
 int32_t plan_fft_stage(int n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, int64_t in_bs, int64_t in_ns,
                        int64_t out_ls, int64_t out_bs, int64_t out_ns, bool inplace, int effort,
                        hipStream_t stream, fft_stage* st, int lds_dma) {
@@ -885,6 +920,17 @@ int32_t plan_fft_stage(int n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, i
                 if (dma_ok(c, d)) cands.push_back(c);
             }
         }
+        // what an untuned stage runs, and both LDS-DMA kernels in their own shape
+        if (lds_dma != 0) {
+            fft_config untuned = cfg;
+            cols_config(untuned, d, inplace, 1);
+            for (const fft_config& c : {untuned, dma_config(cfg, 1), dma_config(cfg, 2)}) {
+                bool known = c.dma && !dma_ok(c, d);
+                for (auto& o : cands)
+                    known |= o.dma == c.dma && o.tpl == c.tpl && o.lpb == c.lpb && o.pad == c.pad && o.radices == c.radices;
+                if (!known) cands.push_back(c);
+            }
+        }
         // each candidate is timed in the form it would run: with the LDS twiddle table where
         // the rule of this configuration gives it one, and at EXHAUSTIVE also in the other form
         for (size_t i = 0, nc = cands.size(); i < nc; i++) {
@@ -921,35 +967,8 @@ int32_t plan_fft_stage(int n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, i
     }
     if (lds_dma == 0) {
         cfg.dma = 0;
-    } else if (!cfg.dma && (lds_dma >= 2 || (!tuned && !dbl))) {
-        // Default for FP32 column-in passes, us per 2 GiB, LDS-DMA (one tile per block) against the
-        // plain column kernel: 16 points 354 / 404, 36 points 384 / 550, 64 points 346 / 395, 210
-        // points 380 / 490, 320 points 374 / 500, 512 points 384 / 442, 900 points 536 / 662; rows
-        // of 210 lines, whose pieces straddle 128-byte lines: 64 points 357 / 441, 320 points 419 /
-        // 514, 512 points 461 / 536.  In place from 48 points on (60 points 394 / 453, 36 points 467 /
-        // 408, 512 points 395 / 453).  Launches of few tiles are bound by latency, where the plain
-        // kernel's loads go straight to the first pass (256 points, 4 MB: 5.9 / 5.2).  FP64 keeps
-        // the plain kernel, which the autotuner preferred there.
-        fft_config c = dma_config(cfg, lds_dma == 2 ? 1 : 2);
-        const bool use = lds_dma >= 2 || (nl * nb >= 8192 && n >= (c.out_cols ? 48 : 16));
-        bool wide = false;
-        if (lds_dma == 1 && !dbl && inplace && cfg.out_cols && n >= 512) {
-            // In-place FP32 column passes of n >= 512 where a 32-line tile (256-byte pieces of
-            // every row) fits with the LDS twiddle table: the plain kernel, persistent, four
-            // butterflies per thread and pass.  EXHAUSTIVE picked it at 512^3 in three runs,
-            // 416 us against 427 us for the LDS-DMA double buffer (the 32-line tile fits only
-            // up to n = 512; at 256^3 and 384^3 the tuner picked other kernels, which keep the
-            // rule below).
-            fft_config w = cfg;
-            const int rmax = *std::max_element(w.radices.begin(), w.radices.end());
-            w.dma = 0;
-            w.lpb = 32;
-            w.pad = 1;
-            w.tpl = std::max(1, n / rmax / 4);
-            apply_twl(w, d, 1);  // the measured form: persistent with LDS twiddles (>= 2048 tiles)
-            if (w.twl && valid(w)) { cfg = w; rec_twl = -1; wide = true; }
-        }
-        if (!wide && use && dma_ok(c, d)) { cfg = c; rec_twl = -1; }
+    } else if (!cfg.dma && (lds_dma >= 2 || !tuned) && cols_config(cfg, d, inplace, lds_dma)) {
+        rec_twl = -1;
     }
     // persistent blocks with the twiddle table in LDS: as the tuning record says (the form it
     // was timed in), else by the rule of the configuration
