@@ -196,13 +196,12 @@ static bool grid_dma_ok(const fft_config& c, const stage_spec& q) {
     return dma_ok(c, make_lines(q.nl, q.nb, q.in_ls, q.in_bs, q.in_ns, q.out_ls, q.out_bs, q.out_ns, c.lpb));
 }
 
-// Candidate tile shapes of a group for the autotuner, the default first: radix schedules of
-// the length (radix_schedules), threads per line of one or two butterflies of the largest
-// radix per pass, and the default's lines per block, halved and doubled.
-static std::vector<fft_config> group_candidates(int n, bool dbl, bool in_cols, bool out_cols, int64_t lines,
-                                                int effort) {
+// Candidate tile shapes of a group for the autotuner, the plain default (base) first: radix
+// schedules of the length (radix_schedules), threads per line of one or two butterflies of the
+// largest radix per pass, and the default's lines per block, halved and doubled.
+static std::vector<fft_config> group_candidates(const fft_config& base, int effort) {
     std::vector<fft_config> out;
-    const fft_config base = default_fft_config(n, dbl, in_cols, out_cols, lines, INT64_MAX);
+    const int n = base.n;
     out.push_back(base);
     const auto scheds = radix_schedules(n, effort >= DTFFT_HIP_EXHAUSTIVE ? 6 : 3);
     for (const auto& r : scheds) {
@@ -231,26 +230,25 @@ static uint64_t fnv1a_ints(const std::vector<int64_t>& v) {
     return h;
 }
 
-// At effort >= MEASURE: time the candidate shapes of one group on scratch buffers and keep the
-// fastest (the project's replacement of dtfft_nvrtc_block_optimizer for the batched cycle).
-// The choice is stored as a tuning record keyed by the group's length, layout and lines.
+// The tile shape of one group in `best`, on entry its plain default; `direct`: the tiles of all of its
+// grids can be loaded into LDS directly.  A tuning record decides, or, at effort >= MEASURE, the
+// candidate that is fastest on scratch buffers (the project's replacement of
+// dtfft_nvrtc_block_optimizer for the batched cycle), else the default rule: FP32 groups load directly
+// where they can.  The choice is stored as a record keyed by the group's length, layout and lines.
 static int32_t tune_group(cycle_t* cy, const std::vector<stage_spec>& specs, const std::vector<int>& members,
-                          bool in_cols, bool out_cols, void* scratch_in, void* scratch_out, fft_config& best,
-                          bool& tuned) {
-    tuned = false;
-    const int n = (int)specs[members[0]].n;
+                          bool direct, void* scratch_in, void* scratch_out, fft_config& best) {
+    const int n = best.n;
+    const fft_config base = best, dma = dma_config(best, 2);
+    if (direct && !cy->dbl) best = dma;
     std::vector<int64_t> sig;
-    int64_t lines = 0;
     for (int g : members) {
         const stage_spec& q = specs[g];
-        lines += q.nl * q.nb;
         sig.insert(sig.end(), {q.nl, q.nb, q.in_ls, q.in_bs, q.in_ns, q.out_ls, q.out_bs, q.out_ns});
     }
     char kb[160];
-    std::snprintf(kb, sizeof kb, "cyc|%d|%c|%d%d|%zu|%016llx", n, cy->dbl ? 'd' : 'f', (int)in_cols, (int)out_cols,
-                  members.size(), (unsigned long long)fnv1a_ints(sig));
+    std::snprintf(kb, sizeof kb, "cyc|%d|%c|%d%d|%zu|%016llx", n, cy->dbl ? 'd' : 'f', (int)base.in_cols,
+                  (int)base.out_cols, members.size(), (unsigned long long)fnv1a_ints(sig));
     const std::string key(kb);
-    best = default_fft_config(n, cy->dbl, in_cols, out_cols, lines, INT64_MAX);
     std::string rec;
     if (tune_lookup(key, rec)) {
         int t, l, p, dm = 0;
@@ -258,21 +256,17 @@ static int32_t tune_group(cycle_t* cy, const std::vector<stage_spec>& specs, con
         std::vector<int> r;
         // "tpl lpb pad radices dma" (records without the last field are of the plain kernel)
         if (std::sscanf(rec.c_str(), "%d %d %d %127s %d", &t, &l, &p, rads, &dm) >= 4 && parse_radices(rads, n, r)) {
-            fft_config c = best;
+            fft_config c = base;
             c.tpl = t; c.lpb = l; c.pad = p; c.radices = r; c.dma = dm == 2 ? 2 : 0;
             bool fits = t * l >= 1 && t * l <= 1024 && fft_lds_bytes(c) <= 160 * 1024;
             if (c.dma) for (int g : members) fits = fits && grid_dma_ok(c, specs[g]);
-            if (fits) { best = c; tuned = true; }
+            if (fits) best = c;
         }
         return DTFFT_HIP_SUCCESS;
     }
     if (cy->effort < DTFFT_HIP_MEASURE || compile_only() || !scratch_in) return DTFFT_HIP_SUCCESS;
-    auto cands = group_candidates(n, cy->dbl, in_cols, out_cols, lines, cy->effort);
-    if (in_cols && global_config().lds_dma != 0) {
-        const fft_config c = dma_config(best, 2);
-        if (std::all_of(members.begin(), members.end(), [&](int g) { return grid_dma_ok(c, specs[g]); }))
-            cands.push_back(c);
-    }
+    auto cands = group_candidates(base, cy->effort);
+    if (direct) cands.push_back(dma);
     // compile the candidates side by side (hipRTC programs are independent)
     {
         std::vector<std::thread> pool;
@@ -311,7 +305,6 @@ static int32_t tune_group(cycle_t* cy, const std::vector<stage_spec>& specs, con
     char buf[160];
     std::snprintf(buf, sizeof buf, "%d %d %d %s %d", best.tpl, best.lpb, best.pad, r.c_str(), best.dma);
     tune_store(key, buf);
-    tuned = true;
     return DTFFT_HIP_SUCCESS;
 }
 
@@ -340,20 +333,20 @@ static int32_t build_stage(cycle_t* cy, int dir, int s, void* scratch_in, void* 
         const stage_spec& sp = specs[members[0]];
         const bool in_cols = sp.in_ns != 1 && sp.in_ls == 1;
         const bool out_cols = sp.out_ns != 1 && sp.out_ls == 1;
-        fft_config cf;
-        bool tuned = false;
-        TRY(tune_group(cy, specs, members, in_cols, out_cols, scratch_in, scratch_out, cf, tuned));
-        std::vector<int> direct;  // grids of the LDS-DMA launch
-        const fft_config cd = dma_config(cf, 2);
-        if (!tuned && in_cols && !cy->dbl && global_config().lds_dma != 0) {
-            for (int g : members) if (grid_dma_ok(cd, specs[g])) direct.push_back(g);
-            members.erase(std::remove_if(members.begin(), members.end(),
-                                         [&](int g) { return grid_dma_ok(cd, specs[g]); }), members.end());
-        }
-        for (const bool dma : {true, false}) {
-            if ((dma ? direct : members).empty()) continue;
+        int64_t lines = 0;
+        for (int g : members) lines += specs[g].nl * specs[g].nb;
+        const fft_config base = default_fft_config((int)sp.n, cy->dbl, in_cols, out_cols, lines, INT64_MAX);
+        // two groups: grids whose tiles can be loaded into LDS directly, and the others
+        std::vector<int> split[2];
+        const fft_config dma = dma_config(base, 2);
+        for (int g : members)
+            split[in_cols && global_config().lds_dma != 0 && grid_dma_ok(dma, specs[g]) ? 0 : 1].push_back(g);
+        for (int i = 0; i < 2; i++) {
+            if (split[i].empty()) continue;
+            fft_config cf = base;
+            TRY(tune_group(cy, specs, split[i], i == 0, scratch_in, scratch_out, cf));
             std::unique_ptr<length_group> grp;
-            TRY(make_group(cy, specs, dma ? direct : members, dma ? cd : cf, grp));
+            TRY(make_group(cy, specs, split[i], cf, grp));
             groups.push_back(std::move(grp));
         }
     }
