@@ -258,7 +258,7 @@ static int32_t tune_group(cycle_t* cy, const std::vector<stage_spec>& specs, con
         if (std::sscanf(rec.c_str(), "%d %d %d %127s %d", &t, &l, &p, rads, &dm) >= 4 && parse_radices(rads, n, r)) {
             fft_config c = base;
             c.tpl = t; c.lpb = l; c.pad = p; c.radices = r; c.dma = dm == 2 ? 2 : 0;
-            bool fits = t * l >= 1 && t * l <= 1024 && fft_lds_bytes(c) <= 160 * 1024;
+            bool fits = t * l >= 1 && t * l <= 1024 && fft_lds_bytes(c) <= 160 * 1024 && (!c.dma || direct);
             if (c.dma) for (int g : members) fits = fits && grid_dma_ok(c, specs[g]);
             if (fits) best = c;
         }

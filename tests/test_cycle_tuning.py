@@ -1,6 +1,8 @@
 """Tuning of the batched cycle's column groups that load LDS directly: a set of grids of which some rows
-allow it is tuned in two groups, and what an untuned cycle runs is among the candidates."""
+allow it is tuned in two groups, what an untuned cycle runs is among the candidates, and a record of
+such a kernel does not overrule lds_dma = 0."""
 import os
+import struct
 import subprocess
 import sys
 
@@ -32,6 +34,30 @@ def kernels(path, effort, grids, lds_dma=1, **env):
                          env=dict(os.environ, **env), capture_output=True, text=True, timeout=110)
     assert out.returncode == 0, out.stderr
     return {ln.split(" ", 1)[1].strip() for ln in out.stdout.splitlines() if ln.startswith("kernel ")}
+
+
+def column_key(grids):
+    """The record key of the forward Y stage of grids with one ny, all of them in one group."""
+    h, mask = 1469598103934665603, (1 << 64) - 1
+    for nx, ny, nz in grids:
+        # nx lines of nz batches; in: lines 1, batches nx ny, elements nx apart; out: ny nz, ny, 1
+        for v in (nx, nz, 1, nx * ny, nx, ny * nz, ny, 1):
+            for b in struct.pack("<q", v):
+                h = ((h ^ b) * 1099511628211) & mask
+    return f"cyc|{grids[0][1]}|f|10|{len(grids)}|{h:016x}"
+
+
+def test_record_keeps_to_lds_dma(tmp_path):
+    if D.device_arch().startswith("gfx950"):
+        pytest.skip("a GPU is present; compile-only behaviour is exercised on CPU hosts")
+    grids = [[64, 96, 48], [32, 96, 80]]
+    for lds_dma, expected in ((1, True), (0, False)):
+        path = tmp_path / str(lds_dma)
+        path.mkdir()
+        (path / "tuning.txt").write_text(f"{column_key(grids)}\t16 16 1 8,12 2\n")  # not the default schedule
+        names = kernels(path, "ESTIMATE", grids, lds_dma, DTFFT_HIP_COMPILE_ONLY="1")
+        assert any("batched_cols_dma_kernel" in k and "Li96ELi8ELi12E" in k for k in names) == expected, names
+        assert any("batched_cols_dma_kernel" in k for k in names) == expected, names
 
 
 @pytest.mark.gpu
