@@ -335,7 +335,7 @@ static int32_t build_stage(cycle_t* cy, int dir, int s, void* scratch_in, void* 
         const bool out_cols = sp.out_ns != 1 && sp.out_ls == 1;
         int64_t lines = 0;
         for (int g : members) lines += specs[g].nl * specs[g].nb;
-        const fft_config base = default_fft_config((int)sp.n, cy->dbl, in_cols, out_cols, lines, INT64_MAX);
+        const fft_config base = default_fft_config((int)sp.n, cy->dbl, in_cols, out_cols, lines, 0);
         // two groups: grids whose tiles can be loaded into LDS directly, and the others
         std::vector<int> split[2];
         const fft_config dma = dma_config(base, 2);

@@ -379,11 +379,11 @@ fft_config default_fft_config(int n, bool dbl, bool in_cols, bool out_cols, int6
         c.pad = 1;
         c.lpb = wide;
         while (!dbl && c.lpb > 8 && (size_t)c.lpb * (size_t)n * (size_t)es > 52 * 1024) c.lpb /= 2;
-        while (c.lpb * 2 * c.tpl <= 128 && c.lpb < 64 && c.lpb < nl) c.lpb *= 2;
+        while (c.lpb * 2 * c.tpl <= 128 && c.lpb < 64 && (nl == 0 || c.lpb < nl)) c.lpb *= 2;
         // half of that for a few lines, where rows of nl lines start on whole 128-byte pieces: else two
         // XCDs share every piece (75 x 128 x 36 FP64, 128 points in place: 4 lines 11.5 us, 8 lines
         // 6.2 us)
-        if (few && nl * es % 128 == 0) while (c.lpb * es > 64 && lines / c.lpb < 512) c.lpb /= 2;
+        if (few && nl > 0 && nl % (128 / es) == 0) while (c.lpb * es > 64 && lines / c.lpb < 512) c.lpb /= 2;
     } else {
         // two waves per block (84 points FP32 on 12 threads: 10 lines 90 us, 5 lines 92 us per
         // 256 MB; FP64 79 and 84 us)

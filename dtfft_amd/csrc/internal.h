@@ -139,7 +139,8 @@ size_t fft_lds_bytes(const fft_config& c);
 // form) for a stage of these lines, and only where the LDS budget allows it.
 void apply_twl(fft_config& c, const lines_desc& d, int mode);
 // Chooses schedule, tpl and lpb for a length and access mode (the default, and the autotuner's
-// first candidate); lines: how many the launch transforms (0: many), nl of them side by side.
+// first candidate); lines: how many the launch transforms (0: many), nl of them side by side (0:
+// not one number, as for the grids of a batched cycle).
 fft_config default_fft_config(int n, bool dbl, bool in_cols, bool out_cols, int64_t lines, int64_t nl);
 void pick_schedule(int n, int points, std::vector<int>& radices, int& tpl);
 std::vector<fft_config> fft_candidates(int n, bool dbl, bool in_cols, bool out_cols, int64_t lines, int64_t nl);
