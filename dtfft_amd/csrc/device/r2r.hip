@@ -28,9 +28,10 @@
 //
 // Powers of two of types 2 and 3 take the persistent fft_r2r_kernel: the real lines go to LDS, the
 // pre-process fills the complex work line in LDS, the Stockham passes of fft_tile run there, and
-// the post-process writes the real outputs.  Every other length whose work length has radices takes
-// r2r_tile_kernel, with any strides.  Both read and write each real element once.  The rest
-// (a prime without a radix in the work length) takes the three launches through a complex buffer.
+// the post-process writes the real outputs.  Every other length whose work length has radices (in
+// FP64 up to 16) takes r2r_tile_kernel, with any strides.  Both read and write each real element once.
+// The rest takes the three launches through a complex buffer, and so do lines that move in place
+// (spaced differently in and out): r2r_tile_kernel orders reads before writes within a block only.
 #include "fft.hip"  // fft_tile: the Stockham passes, here run on work lines held in LDS
 
 struct r2r_desc {

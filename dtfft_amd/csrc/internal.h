@@ -224,8 +224,8 @@ struct r2r_stage {
     int32_t init_cols(int kind, int64_t n, bool dbl, int64_t nl, int64_t nb, int64_t in_bs, int64_t in_es,
                       int64_t out_ls, int64_t out_bs, int64_t out_es, bool out_cols, bool* ok);
     // One launch of r2r_tile_kernel for any strides on both sides (in place where they are equal);
-    // *ok is false (nothing set up) where the work length has a prime without a radix or the
-    // tile does not fit.
+    // *ok is false (nothing set up) where the work length has a prime without a radix, in FP64 one
+    // above 13, or the tile does not fit.
     int32_t init_tile(int kind, int64_t n, bool dbl, int64_t nl, int64_t nb, int64_t in_ls, int64_t in_bs,
                       int64_t in_es, int64_t out_ls, int64_t out_bs, int64_t out_es, bool* ok);
     // Chunk-blocked pair (fused kernels, half-length form): `rows` writing its lines (nl

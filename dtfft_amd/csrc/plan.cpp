@@ -250,7 +250,7 @@ static int32_t build_r2r(plan_t* p) {
     // Fused sequence, as the fused C2C one: forward X rows, X->Y + Y, Y->Z + Z; backward Z
     // rows, Z->X + X, Y in place on the X-pencil (the axes of a separable R2R commute).  Taken
     // when every stage that reads across lines has the fused form (types 2 / 3 of even length,
-    // lines in whole 128-byte tile rows); otherwise the reference's sequence with permutes.
+    // lines in whole 128-byte tile rows); otherwise the general column stages below.
     if (p->fused) {
         const int k0 = p->kind[0], k1 = p->kind[1];
         const int i0 = r2r_inverse_kind(k0), i1 = r2r_inverse_kind(k1);

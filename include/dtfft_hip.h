@@ -171,18 +171,21 @@ int32_t dtfft_hip_kernel_destroy(void* handle);
  * r2r_kinds is required for FFT_R2R (dtFFT kind ids, include/dtfft_config.h.in:66-73), one per
  * dimension in fft_sizes order; FFTW semantics, unnormalised.  The forward sign applies the
  * kinds, the backward sign their inverses (src/dtfft_utils.F90:447-471).  An R2R stage runs
- * a complex FFT of length n, 2n (type 4), 2(n-1) (DCT-1) or 2(n+1) (DST-1).
- * Any length is accepted, as cuFFT and FFTW accept it: lengths whose primes are <= 13 run
- * the mixed-radix kernels, others Bluestein's chirp z-transform, odd R2C/C2R lengths a
- * direct odd-length kernel.  A length whose work line (n, or the Bluestein length >= 2n-1)
- * exceeds the 160 KiB of LDS of one workgroup returns DTFFT_HIP_ERROR_UNSUPPORTED_SIZE. */
+ * a complex FFT of length n/2 (types 2 to 4 of even n), n (types 2 and 3 of odd n), 2n (type 4
+ * of odd n), n-1 (DCT-1) or n+1 (DST-1).
+ * Any length is accepted, as cuFFT and FFTW accept it: lengths whose primes are <= 13, or up to
+ * 61 (FP32) and 37 (FP64) where the Bluestein length below would fit, run the mixed-radix
+ * kernels, others Bluestein's chirp z-transform, odd R2C/C2R lengths with primes <= 13 a direct
+ * odd-length kernel.  A length whose work line (n, or the Bluestein length >= 2n-1; R2R: the
+ * whole extension of n, 2n, 2(n-1) or 2(n+1) points) exceeds the 160 KiB of LDS of one workgroup
+ * returns DTFFT_HIP_ERROR_UNSUPPORTED_SIZE. */
 int32_t dtfft_hip_fft_create(int8_t fft_rank, int8_t fft_type, int32_t precision, int32_t idist,
                              int32_t odist, int32_t how_many, const int32_t* fft_sizes,
                              const int32_t* inembed, const int32_t* onembed,
                              const int32_t* r2r_kinds, int32_t effort, void* stream, void** plan);
 /* Replaces abstract_executor%execute_private: sign = FFT_FORWARD (-1) or FFT_BACKWARD (+1).
  * For R2C, forward is real->complex and backward complex->real (in != out required).
- * R2R may run in place. */
+ * R2R may run in place, also with idist != odist. */
 int32_t dtfft_hip_fft_execute(void* plan, const void* in, void* out, int8_t sign);
 int32_t dtfft_hip_fft_destroy(void* plan);
 
@@ -203,13 +206,13 @@ typedef struct {
     int32_t lds_dma;              /* column-in FFT passes through LDS tiles filled by direct global->LDS
                                      loads: 0 never, 1 where the autotuner (or the default rule) picks
                                      them (default), 2 the double-buffer kernel wherever the stage shape
-                                     allows, 3 the single-buffer kernel (one tile per block, two
-                                     blocks per CU) likewise */
+                                     allows, 3 the single-buffer kernel (one tile per block,
+                                     several blocks per CU) likewise */
     int32_t twl;                  /* FFT kernels that keep the twiddle table in LDS (persistent blocks):
                                      0 never, 1 where the default rule picks them (default: FP32 rows
-                                     of n >= 2048, FP32 column-in passes without LDS-DMA, the fused
-                                     C2R, on stages of >= 2048 tiles), 2 every stage whose kernel has
-                                     the form and whose LDS budget allows it */
+                                     of n > 1024 while two blocks fit a CU, FP32 column-in passes
+                                     without LDS-DMA, on stages of >= 2048 tiles), 2 every stage whose
+                                     kernel has the form and whose LDS budget allows it */
     int32_t blocked;              /* 1 (default): a row FFT pass whose output the next pass reads as
                                      column tiles writes it chunk-blocked (each tile's lines as one
                                      contiguous block), so that the column pass streams it; the
